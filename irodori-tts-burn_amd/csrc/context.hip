@@ -376,7 +376,7 @@ int ensure_nvec(irodori_ctx* c, int nvec) {
 // vectors already in c->cond): tab[v][l][k][ch][:].  With the fused adaLN also the shift
 // biases of layers [l0, l1) (whose weights must be loaded; all layers by default):
 // biasq[l][v] = shift_attn(v, l) W_qkvg, bias13[l][v] = shift_mlp(v, l) W13.
-int enqueue_mod_table(irodori_ctx* c, int nvec, bool skip_mlp, int l0 = 0, int l1 = -1) {
+int enqueue_mod_table(irodori_ctx* c, int nvec, bool skip_mlp, bool shift = true, int l0 = 0, int l1 = -1) {
     const auto& g = c->cfg;
     int D = g.model_dim, L = g.num_layers, r = g.adaln_rank;
     if (l1 < 0) l1 = L;
@@ -961,6 +961,20 @@ int irodori_ctx_create(int device, const irodori_dit_config* cfg, irodori_ctx** 
     c->layers.resize(L);
     int ntl = (T + 63) / 64;
     int Tp = ntl * 64, Sp = (S + 63) / 64 * 64;
+    // Every layer's context and k_norm in one allocation each, layer after layer: the device
+    // build writes all layers of a row in one launch.
+    const size_t nk = (size_t)R * H * T * Dh, nv = (size_t)R * H * Dh * Tp;
+    char *ctx_k = nullptr, *ctx_v = nullptr;
+    float *ctx_mask = nullptr, *k_norm = nullptr;
+    int* tile_on = nullptr;
+    unsigned long long* tile_bits = nullptr;
+    IRO_TRY(dalloc(c.get(), &ctx_k, es * L * nk));
+    IRO_TRY(dalloc(c.get(), &ctx_v, es * L * nv));
+    IRO_HIP_CHECK(hipMemsetAsync(ctx_v, 0, es * L * nv, c->stream));
+    IRO_TRY(dalloc(c.get(), &ctx_mask, sizeof(float) * L * (size_t)R * T));
+    IRO_TRY(dalloc(c.get(), &tile_on, sizeof(int) * L * (size_t)R * ntl));
+    IRO_TRY(dalloc(c.get(), &tile_bits, sizeof(unsigned long long) * L * (size_t)R * ntl));
+    IRO_TRY(dalloc(c.get(), &k_norm, sizeof(float) * L * (size_t)H * Dh));
     for (int l = 0; l < L; l++) {
         auto& lb = c->layers[l];
         const size_t wes = c->fp8 ? 1 : es;  // weight element bytes
@@ -975,19 +989,18 @@ int irodori_ctx_create(int device, const irodori_dit_config* cfg, irodori_ctx** 
             IRO_TRY(dalloc(c.get(), &lb.ws_2, sizeof(float) * D));
         }
         IRO_TRY(dalloc(c.get(), &lb.q_norm, sizeof(float) * H * Dh));
-        IRO_TRY(dalloc(c.get(), &lb.k_norm, sizeof(float) * H * Dh));
+        lb.k_norm = k_norm + (size_t)l * H * Dh;
         for (int k = 0; k < 2; k++)
             for (int ch = 0; ch < 3; ch++) {
                 IRO_TRY(dalloc(c.get(), &lb.ada_down[k][ch], sizeof(float) * (size_t)D * g.adaln_rank));
                 IRO_TRY(dalloc(c.get(), &lb.ada_up[k][ch], sizeof(float) * (size_t)g.adaln_rank * D));
                 IRO_TRY(dalloc(c.get(), &lb.ada_up_b[k][ch], sizeof(float) * D));
             }
-        IRO_TRY(dev_alloc(c.get(), &lb.ctx_k, es * (size_t)R * H * T * Dh));
-        IRO_TRY(dev_alloc(c.get(), &lb.ctx_v, es * (size_t)R * H * Dh * Tp));
-        IRO_HIP_CHECK(hipMemsetAsync(lb.ctx_v, 0, es * (size_t)R * H * Dh * Tp, c->stream));
-        IRO_TRY(dalloc(c.get(), &lb.ctx_mask, sizeof(float) * (size_t)R * T));
-        IRO_TRY(dalloc(c.get(), &lb.tile_on, sizeof(int) * (size_t)R * ntl));
-        IRO_TRY(dalloc(c.get(), &lb.tile_bits, sizeof(unsigned long long) * (size_t)R * ntl));
+        lb.ctx_k = ctx_k + es * l * nk;
+        lb.ctx_v = ctx_v + es * l * nv;
+        lb.ctx_mask = ctx_mask + (size_t)l * R * T;
+        lb.tile_on = tile_on + (size_t)l * R * ntl;
+        lb.tile_bits = tile_bits + (size_t)l * R * ntl;
         lb.row_set.assign(R, 0);
     }
     IRO_TRY(dalloc(c.get(), &c->cond_w0, sizeof(float) * (size_t)g.timestep_embed_dim * D));
@@ -1201,13 +1214,18 @@ int irodori_load_ctx_proj_weights(irodori_ctx* c, int layer, int text_dim, int a
         const int K = dims[sgm];
         if (K == 0) continue;
         const int kpad = (K + 63) / 64 * 64;
-        if (!lb.w_ctx[sgm]) IRO_TRY(dev_alloc(c, &lb.w_ctx[sgm], c->esz * (size_t)2 * HD * kpad));
+        if (!lb.w_ctx[sgm]) {  // every layer's in one allocation, so the build is one GEMM over all of them
+            char* w_all = nullptr;
+            const size_t layer_bytes = c->esz * (size_t)2 * HD * kpad;
+            IRO_TRY(dalloc(c, &w_all, layer_bytes * g.num_layers));
+            for (int l = 0; l < g.num_layers; l++) c->layers[l].w_ctx[sgm] = w_all + l * layer_bytes;
+        }
         const float* src[2] = {sgm ? w->wk_aux : w->wk_text, sgm ? w->wv_aux : w->wv_text};
         std::vector<float> padded((size_t)kpad * HD, 0.f);  // Burn [d_in, kv_dim], rows past d_in zero
         for (int kv = 0; kv < 2; kv++) {
             memcpy(padded.data(), src[kv], sizeof(float) * (size_t)K * HD);
             IRO_TRY(ingest_kmajor(c, padded.data(), kpad, HD, 0,
-                                  static_cast<char*>(lb.w_ctx[sgm]) + c->esz * (size_t)kv * HD * kpad));
+                                  static_cast<char*>(lb.w_ctx[sgm]) + c->esz * (size_t)kv * HD * kpad, true));
         }
         c->ctx_dim[sgm] = K;
         c->ctx_kpad[sgm] = kpad;
@@ -1247,75 +1265,67 @@ int irodori_build_ctx_kv(irodori_ctx* c, int row, int t_text, const float* text_
     IRO_HIP_CHECK(hipSetDevice(c->device));
     const int T1 = g.max_ctx > 0 ? g.max_ctx : 1, vs1 = (T1 + 63) / 64 * 64;
 
-    // States -> compute dtype, input dim zero-padded, staged [text rows | aux rows].
+    // States f32 -> compute dtype, input dim zero-padded, staged [text rows | aux rows], with the
+    // caller's f32 rows and the key mask staged behind them.
     const int lens[2] = {t_text, t_aux};
     const float* states[2] = {text_state, aux_state};
-    size_t off[2], total = 0;
-    for (int sgm = 0; sgm < 2; sgm++) {
-        off[sgm] = total;
-        if (lens[sgm]) total += (size_t)lens[sgm] * c->ctx_kpad[sgm];
-    }
+    const size_t kmax = std::max(c->ctx_kpad[0], c->ctx_kpad[1]), half = (size_t)T1 * kmax;
     if (!c->ctx_state) {  // t_text + t_aux <= max_ctx rows of the wider padded input
-        const int kmax = c->ctx_kpad[0] > c->ctx_kpad[1] ? c->ctx_kpad[0] : c->ctx_kpad[1];
-        c->ctx_state_bytes = (size_t)T1 * kmax * c->esz;
+        c->ctx_state_bytes = half * (c->esz + sizeof(float)) + T1;
         IRO_TRY(dev_alloc(c, &c->ctx_state, c->ctx_state_bytes));
     }
-    IRO_REQUIRE(total * c->esz <= c->ctx_state_bytes, IRODORI_ERR_SHAPE, "context states exceed the staging buffer");
-    std::vector<float> sf(total, 0.f);
-    for (int sgm = 0; sgm < 2; sgm++)
-        for (int j = 0; j < lens[sgm]; j++)
-            memcpy(sf.data() + off[sgm] + (size_t)j * c->ctx_kpad[sgm], states[sgm] + (size_t)j * c->ctx_dim[sgm],
-                   sizeof(float) * c->ctx_dim[sgm]);
-    std::vector<uint16_t> sb;
-    if (c->bf16) {
-        sb.resize(total);
-        for (size_t i = 0; i < total; i++) sb[i] = bf16_bits(sf[i]);
-        IRO_TRY(upload(c, c->ctx_state, sb.data(), total * 2));
-    } else if (total) {
-        IRO_TRY(upload(c, c->ctx_state, sf.data(), total * 4));
+    IRO_REQUIRE(half * (c->esz + sizeof(float)) + T1 <= c->ctx_state_bytes, IRODORI_ERR_SHAPE,
+                "context states exceed the staging buffer");
+    char* const operand = static_cast<char*>(c->ctx_state);
+    float* const raw = reinterpret_cast<float*>(operand + half * c->esz);
+    uint8_t* const d_mask = reinterpret_cast<uint8_t*>(raw + half);
+    size_t off[2] = {0, 0}, roff = 0, total = 0;
+    for (int sgm = 0; sgm < 2; sgm++) {
+        const int n = lens[sgm], dim = c->ctx_dim[sgm], kpad = c->ctx_kpad[sgm];
+        off[sgm] = total;
+        if (n == 0) continue;
+        IRO_TRY(upload(c, raw + roff, states[sgm], sizeof(float) * (size_t)n * dim));
+        if (c->bf16)
+            launch_ctx_states<bf16>(raw + roff, n, dim, kpad, reinterpret_cast<bf16*>(operand) + total, c->stream);
+        else
+            launch_ctx_states<float>(raw + roff, n, dim, kpad, reinterpret_cast<float*>(operand) + total, c->stream);
+        roff += (size_t)n * dim;
+        total += (size_t)n * kpad;
     }
-    IRO_HIP_CHECK(hipStreamSynchronize(c->stream));  // the host staging vectors end here
-    std::vector<uint8_t> mask(t_ctx);
-    for (int j = 0; j < t_text; j++) mask[j] = text_mask[j] ? 1 : 0;
-    for (int j = 0; j < t_aux; j++) mask[t_text + j] = aux_mask[j] ? 1 : 0;
+    if (t_text) IRO_TRY(upload(c, d_mask, text_mask, t_text));
+    if (t_aux) IRO_TRY(upload(c, d_mask + t_text, aux_mask, t_aux));
 
-    for (int l = 0; l < L; l++) {
-        auto& lb = c->layers[l];
-        const size_t nk = (size_t)H * T1 * Dh, nv = (size_t)H * Dh * vs1;
-        char* ck = static_cast<char*>(lb.ctx_k) + (size_t)row * nk * c->esz;
-        char* cv = static_cast<char*>(lb.ctx_v) + (size_t)row * nv * c->esz;
-        // Keys past t_ctx (and the V^T padding) hold zeros, as after irodori_set_ctx_kv.
-        IRO_HIP_CHECK(hipMemsetAsync(ck, 0, nk * c->esz, c->stream));
-        IRO_HIP_CHECK(hipMemsetAsync(cv, 0, nv * c->esz, c->stream));
+    const int R = g.max_rows, ntl = vs1 / 64;
+    const size_t nk = (size_t)H * T1 * Dh, nv = (size_t)H * Dh * vs1;
+    auto& l0 = c->layers[0];
+    auto build = [&](auto tag) -> int {
+        typedef decltype(tag) T;
+        T* const ck = static_cast<T*>(l0.ctx_k) + row * nk;
+        T* const cv = static_cast<T*>(l0.ctx_v) + row * nv;
         for (int sgm = 0; sgm < 2; sgm++) {
             if (lens[sgm] == 0) continue;
-            int rc;
-            if (c->bf16) {
-                GemmArgs<bf16> ga{};
-                ga.A = static_cast<const bf16*>(c->ctx_state) + off[sgm];
-                ga.W = static_cast<const bf16*>(lb.w_ctx[sgm]);
-                ga.M = lens[sgm]; ga.N = 2 * HD; ga.K = c->ctx_kpad[sgm]; ga.S = lens[sgm];
-                ga.H = H; ga.D = g.model_dim; ga.eps = g.norm_eps; ga.k_norm = lb.k_norm;
-                ga.Ck = reinterpret_cast<bf16*>(ck); ga.Cv = reinterpret_cast<bf16*>(cv);
-                ga.key_off = sgm ? t_text : 0; ga.ctx_stride = T1; ga.ctx_vstride = vs1;
-                rc = launch_gemm<bf16>(EPI_CTXKV, ga, c->stream);
-            } else {
-                GemmArgs<float> ga{};
-                ga.A = static_cast<const float*>(c->ctx_state) + off[sgm];
-                ga.W = static_cast<const float*>(lb.w_ctx[sgm]);
-                ga.M = lens[sgm]; ga.N = 2 * HD; ga.K = c->ctx_kpad[sgm]; ga.S = lens[sgm];
-                ga.H = H; ga.D = g.model_dim; ga.eps = g.norm_eps; ga.k_norm = lb.k_norm;
-                ga.Ck = reinterpret_cast<float*>(ck); ga.Cv = reinterpret_cast<float*>(cv);
-                ga.key_off = sgm ? t_text : 0; ga.ctx_stride = T1; ga.ctx_vstride = vs1;
-                rc = launch_gemm<float>(EPI_CTXKV, ga, c->stream);
+            GemmArgs<T> ga{};
+            ga.A = reinterpret_cast<const T*>(operand) + off[sgm];
+            ga.W = static_cast<const T*>(l0.w_ctx[sgm]);
+            ga.w_tiled = 1;
+            ga.M = lens[sgm]; ga.N = L * 2 * HD; ga.K = c->ctx_kpad[sgm]; ga.S = lens[sgm];
+            ga.H = H; ga.D = g.model_dim; ga.eps = g.norm_eps; ga.k_norm = l0.k_norm;
+            ga.Ck = ck; ga.Cv = cv; ga.ck_layer = R * nk; ga.cv_layer = R * nv;
+            ga.key_off = sgm ? t_text : 0; ga.ctx_stride = T1; ga.ctx_vstride = vs1;
+            if (launch_gemm<T>(EPI_CTXKV, ga, c->stream)) {
+                set_last_error("context KV gemm shape");
+                return IRODORI_ERR_SHAPE;
             }
-            if (rc) { set_last_error("context KV gemm shape"); return IRODORI_ERR_SHAPE; }
         }
-        IRO_TRY(check_launch("context KV build"));
-        IRO_TRY(upload_row_mask(c, lb, row, t_ctx, mask.data()));
-        lb.row_set[row] = 1;
-    }
-    IRO_HIP_CHECK(hipStreamSynchronize(c->stream));
+        // Keys past t_ctx (and the V^T padding) hold zeros, as after irodori_set_ctx_kv.
+        launch_ctx_finish<T>(ck, cv, R * nk, R * nv, d_mask, l0.ctx_mask + (size_t)row * T1,
+                             l0.tile_on + (size_t)row * ntl, l0.tile_bits + (size_t)row * ntl, (size_t)R * T1,
+                             (size_t)R * ntl, L, H, Dh, t_ctx, T1, vs1, vt_bf16_order(c), c->stream);
+        return check_launch("context KV build");
+    };
+    IRO_TRY(c->bf16 ? build(bf16()) : build(float()));
+    IRO_HIP_CHECK(hipStreamSynchronize(c->stream));  // the caller's host buffers are free from here on
+    for (auto& lb : c->layers) lb.row_set[row] = 1;
     if (c->t_ctx != t_ctx) {
         c->graphs.clear();
     }

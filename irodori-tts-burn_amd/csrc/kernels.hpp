@@ -162,6 +162,20 @@ void launch_scale_ctx_aux(const T* src_k, const T* src_v, T* dst_k, T* dst_v, in
                           int aux_start, float factor, hipStream_t st);
 void launch_scale_copy(const float* src, float* dst, int n, float s, hipStream_t st);
 
+// Context states [rows, dim] f32 -> the projections' operand [rows, kpad] in T, columns past
+// dim zero.
+template <typename T>
+void launch_ctx_states(const float* src, int rows, int dim, int kpad, T* dst, hipStream_t st);
+// One row's context of every layer past its t_ctx keys, and its mask (nonzero bytes attend):
+// K rows and V^T columns t_ctx .. zeroed (K [H, T1, Dh], V^T [H, Dh, vs1] at vt_pos_bf16 with
+// bf16_order, else vt_pos_f32; layer strides nk / nv elements), the float mask [T1], the
+// per-tile flags and the 64-bit validity words (ntl per row; layer strides mask_layer /
+// tile_layer elements).
+template <typename T>
+void launch_ctx_finish(T* K, T* V, size_t nk, size_t nv, const uint8_t* mask, float* fmask, int* tile_on,
+                       unsigned long long* bits, size_t mask_layer, size_t tile_layer, int layers, int H, int Dh,
+                       int t_ctx, int T1, int vs1, bool bf16_order, hipStream_t st);
+
 // ---- kernels_ops.hip -------------------------------------------------------------------
 // The joint-attention operator's staging: latent q, k, v [B, S, H, 64] f32 and gate logits
 // [B, S, H*64] f32 (nullable: gate 1) into the layouts the QKV+gate epilogue writes -- Q
@@ -231,12 +245,15 @@ struct GemmArgs {
     const float* rope_cs;   // [S, Dh/2, 2]: the same (cos, sin) pairs interleaved
     int H, D;
     float eps;
-    // EPI_CTXKV (context KV build, attention.rs:431-501): N = 2 H Dh columns [K | V] of the
-    // context rows key_off .. key_off + M - 1: K head-normed with k_norm into Ck
-    // [H, ctx_stride, Dh], V into Cv = V^T [H, Dh, ctx_vstride] at vt_pos_bf16 / vt_pos_f32.
+    // EPI_CTXKV (context KV build, attention.rs:431-501): the 2 H Dh columns [K | V] of every
+    // layer side by side, N = layers * 2 H Dh, for the context rows key_off .. key_off + M - 1:
+    // K head-normed with k_norm [layers, H, Dh] into Ck [H, ctx_stride, Dh], V into Cv = V^T
+    // [H, Dh, ctx_vstride] at vt_pos_bf16 / vt_pos_f32; layer l's Ck / Cv lie l * ck_layer /
+    // l * cv_layer elements further on.  D = H Dh.
     T* Ck;
     T* Cv;
     int key_off, ctx_stride, ctx_vstride;
+    size_t ck_layer, cv_layer;
     // EPI_ADD: x[m, n] = (x[m, n] + acc) * rmask[m] (rmask nullable: 1), the encoder's
     // plain residual with its per-block re-masking (text_encoder.rs:131-145).
     const float* rmask;

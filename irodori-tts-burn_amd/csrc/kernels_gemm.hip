@@ -918,13 +918,16 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
         // 64-dim heads) or the 16x16 attention's (f32, and 128-dim heads).
         constexpr int Dh = WN;
         const int HD = a.H * Dh;
-        const int col0 = n0 + wn0;
+        const int layer = (n0 + wn0) / (2 * HD);
+        const int col0 = n0 + wn0 - layer * 2 * HD;
         const bool is_k = col0 < HD;
         const int h = (is_k ? col0 : col0 - HD) / Dh;
+        T* const Ck = a.Ck + layer * a.ck_layer;
+        T* const Cv = a.Cv + layer * a.cv_layer;
         if (is_k) {
             float nw[FN];
 #pragma unroll
-            for (int j = 0; j < FN; j++) nw[j] = a.k_norm[h * Dh + 32 * j + cl];
+            for (int j = 0; j < FN; j++) nw[j] = a.k_norm[layer * HD + h * Dh + 32 * j + cl];
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
@@ -936,7 +939,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
                     const float ss = half_wave_sum(sq);
                     const float inv = __builtin_amdgcn_rsqf(ss * (1.f / (float)Dh) + a.eps);
                     if (row >= a.M) continue;
-                    T* o = a.Ck + ((size_t)h * a.ctx_stride + a.key_off + row) * Dh;
+                    T* o = Ck + ((size_t)h * a.ctx_stride + a.key_off + row) * Dh;
 #pragma unroll
                     for (int j = 0; j < FN; j++) o[32 * j + cl] = from_f32<T>(acc[i][j][e] * inv * nw[j]);
                 }
@@ -951,7 +954,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
                     const int pos = (sizeof(T) == 2 && Dh == 64) ? vt_pos_bf16(key) : vt_pos_f32(key);
 #pragma unroll
                     for (int j = 0; j < FN; j++)
-                        a.Cv[((size_t)h * Dh + 32 * j + cl) * a.ctx_vstride + pos] = from_f32<T>(acc[i][j][e]);
+                        Cv[((size_t)h * Dh + 32 * j + cl) * a.ctx_vstride + pos] = from_f32<T>(acc[i][j][e]);
                 }
         }
     } else if constexpr (EPI == EPI_QKVG && WN == 128) {
@@ -1283,7 +1286,7 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
                 return -1;
             break;
         case EPI_CTXKV:
-            if (!a.Ck || !a.Cv || !a.k_norm || a.H <= 0 || a.N != 2 * a.H * (BN / WAVES_N)) return -1;
+            if (!a.Ck || !a.Cv || !a.k_norm || a.H <= 0 || a.D != a.H * (BN / WAVES_N) || a.N % (2 * a.D)) return -1;
             break;
     }
     // Fused adaLN: a consumer takes bf16 / f32 operands of the QKVG or SwiGLU projections
@@ -1379,7 +1382,7 @@ int launch_gemm(int epi, const GemmArgs<T>& a, hipStream_t st) {
             if (a.H > 0 && a.D == a.H * 128) return launch_cfg<T, 128, 128, 4, 1, 2, EPI_QKVG>(a, st);
             return launch_cfg<T, 128, 128, 2, 2, 2, EPI_QKVG>(a, st);
         case EPI_CTXKV:
-            if (a.H > 0 && a.N == 2 * a.H * 128) return launch_cfg<T, 128, 128, 4, 1, 2, EPI_CTXKV>(a, st);
+            if (a.H > 0 && a.D == a.H * 128) return launch_cfg<T, 128, 128, 4, 1, 2, EPI_CTXKV>(a, st);
             return launch_cfg<T, 128, 128, 2, 2, 2, EPI_CTXKV>(a, st);
     }
     return -1;

@@ -449,30 +449,23 @@ int irodori_op_fused_adaln(const float* x, const float* scale, const float* shif
  * q [B,H,Sq,Dh], k/v [B,H,Skv,Dh] in `dtype` (F32, BF16 or F16: native_fa_sdpa_f16_in's
  * f16 storage, f32 accumulation), mask [B,Skv] f32 with 1.0 = attend (values < 0.5 mask
  * the key; may be NULL), out [B,H,Sq,Dh] f32.  Dh in {64, 128}.  A fully masked query row
- * yields 0.  Enqueued on `stream` without waiting.  With Dh = 64, a 16-bit dtype and
- * seq_kv <= 16384 the call stages Q (pre-scaled), V^T and the key bits in a device buffer it
- * allocates and frees in stream order on `stream` (hipMallocAsync / hipFreeAsync), and runs
- * the model's joint attention kernel on them; other shapes need no staging and run the
- * generic flash kernel, whose softmax is f32 throughout.  Precision of the staged path: the
- * scores and the softmax state are f32, but q * scale * log2(e) and the probabilities P
- * (the P V MFMA operand) are rounded to the operand dtype, as the model's bf16 attention
- * does; the reference's native FA kernels keep both in f32.  Measured against a float64
- * SDPA of the same rounded inputs at config 2's shape: 2.4e-3 relative L2 in bf16 and
- * 3.0e-4 in f16 (bars 1e-2 and 2e-3; max abs 1.5e-3 and 2.0e-4). */
+ * yields 0.  Enqueued on `stream` without waiting, with no device memory of its own.  The
+ * scores and the softmax state are f32; the probabilities P (the P V MFMA operand) are rounded
+ * to the operand dtype in the 16-bit forms, where the reference's native FA kernels keep them
+ * in f32.  Measured against a float64 SDPA of the same rounded inputs at 2 x 16 heads x 750 x
+ * 1381: 1.6e-3 relative L2 in bf16 and 2.0e-4 in f16. */
 int irodori_op_sdpa(int dtype, const void* q, const void* k, const void* v, const float* mask,
                     int batch, int heads, int seq_q, int seq_kv, int head_dim, float scale,
                     float* out, void* stream);
 /* No counterpart in the reference: irodori_op_sdpa for callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops that forbid hipMalloc).  Same
- * arguments, kernels and results; the staging of the 16-bit head_dim-64 path lives in one
- * fixed device buffer of IRODORI_SDPA_SCRATCH_BYTES per GPU, held until the process ends,
- * instead of a per-call allocation.  A shape whose staging (Q + V^T in the operand dtype +
- * the key bits, each rounded up to 256 bytes) exceeds it returns IRODORI_ERR_SHAPE.  Every
- * call on a GPU shares that buffer: calls that overlap on one GPU (other streams or
- * threads) race.  `stream` must belong to the current device (else IRODORI_ERR_INVALID_ARG).
- * The first call on a device looks up the buffer's address and must not be made under graph
- * capture (IRODORI_ERR_INVALID_ARG): capturing callers make one call outside the capture
- * first; later calls may be captured and replayed. */
+ * arguments, kernels and results.  With a 16-bit dtype, head_dim 64 and seq_kv <= 16384 it
+ * takes operands of at most IRODORI_SDPA_SCRATCH_BYTES (Q + V^T with its keys rounded up to 64,
+ * in the operand dtype, + one key bit each, every part rounded up to 256 bytes; else
+ * IRODORI_ERR_SHAPE), `stream` must belong to the current device (else
+ * IRODORI_ERR_INVALID_ARG), and the first call on a device, which loads the kernel, must not be
+ * made under graph capture (IRODORI_ERR_INVALID_ARG): capturing callers make one call outside
+ * the capture first; later calls may be captured and replayed. */
 #define IRODORI_SDPA_SCRATCH_BYTES (16u << 20)
 int irodori_op_sdpa_noalloc(int dtype, const void* q, const void* k, const void* v, const float* mask,
                             int batch, int heads, int seq_q, int seq_kv, int head_dim, float scale,

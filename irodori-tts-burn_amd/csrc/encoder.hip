@@ -144,7 +144,11 @@ int enc_block(irodori_encoder* e, const EncLayer& L, int B, int S) {
     aa.out_mode = 0;
     aa.G = static_cast<const T*>(e->gate);
     aa.O = static_cast<T*>(e->o);
-    const int arc = Dh == 64 ? launch_attention<T, 64>(aa, e->stream) : launch_attention<T, 128>(aa, e->stream);
+    int arc;
+    if constexpr (sizeof(T) == 2)
+        arc = Dh == 64 ? launch_attention_nv<T, 64>(aa, e->stream) : launch_attention_nv<T, 128>(aa, e->stream);
+    else
+        arc = Dh == 64 ? launch_attention<T, 64>(aa, e->stream) : launch_attention<T, 128>(aa, e->stream);
     IRO_REQUIRE(arc == 0, IRODORI_ERR_SHAPE, "encoder attention rejected the shape");
     IRO_TRY(enc_gemm<T>(e, EPI_ADD, static_cast<const T*>(e->o), L.w_o, M, E, E, nullptr, e->x, nullptr, nullptr));
     launch_rmsnorm_w<T>(e->x, L.mlp_norm, M, E, g.norm_eps, h, E, e->stream);

@@ -29,67 +29,23 @@
 // softmax of the current one.
 #include <type_traits>
 
-#include "common.hpp"
+#include "attn_util.hpp"
 #include "kernels.hpp"
 
 namespace irodori {
 
 namespace {
 
-// Max of v over lanes l and l ^ 32 (the two halves of a query column) by v_permlane32_swap,
-// a VALU exchange, instead of an LDS-routed shuffle.
-__device__ __forceinline__ float max_halves(float v) {
-    const unsigned u = __builtin_bit_cast(unsigned, v);
-    const auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return fmaxf(__builtin_bit_cast(float, (unsigned)sw[0]), __builtin_bit_cast(float, (unsigned)sw[1]));
-}
-// Sum of v over lanes l and l ^ 32, the same exchange (the same value in both lanes).
-__device__ __forceinline__ float sum_halves(float v) {
-    const unsigned u = __builtin_bit_cast(unsigned, v);
-    const auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return __builtin_bit_cast(float, (unsigned)sw[0]) + __builtin_bit_cast(float, (unsigned)sw[1]);
-}
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
-// 8-element operand vector of the 32x32x16 matrix-core step for each element type.
-template <typename T>
-struct Vec8;
-template <>
-struct Vec8<bf16> {
-    typedef bf16x8 type;
-};
-template <>
-struct Vec8<f16> {
-    typedef f16x8 type;
-};
-__device__ __forceinline__ f32x16 mma32x16(bf16x8 a, bf16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x16 mma32x16(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
 constexpr int KT = 64;
 constexpr int TILE_BYTES = KT * 128;  // 64 rows x 128 bytes (bf16 Dh = 64)
 constexpr float TAU = 16.0f;          // lazy-reference slack, log2 units
 constexpr float kSumMax = (float)(1u << (int)TAU);  // a lane's tile sum above it moves the reference
 
-__device__ __forceinline__ void raw_barrier() { asm volatile("s_barrier" ::: "memory"); }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, unsigned bytes) {
-    // Raw (stride 0) buffer; dword3 0x00020000 is the gfx9-family data format for raw access.
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ void buf_load_lds16(__amdgpu_buffer_rsrc_t r, unsigned voff, void* lds) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
-}
 __device__ __forceinline__ int swz(int r, int c) { return c ^ ((r >> 1) & 7); }
 template <typename T>
 __device__ __forceinline__ typename Vec8<T>::type frag(const unsigned char* tile, int r, int chunk) {
     return *reinterpret_cast<const typename Vec8<T>::type*>(tile + r * 128 + (swz(r, chunk) << 4));
 }
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // x rounded to the operand type (the softmax reference must be exactly representable).
 template <typename T>
 __device__ __forceinline__ float round_to(float x) { return static_cast<float>(static_cast<T>(x)); }
@@ -598,92 +554,8 @@ int launch_attention32_t(const AttnArgs<T>& a, hipStream_t st) {
     return launch_attn32_cfg<T, 2, 2, 4>(a, st);
 }
 
-// Operator staging (irodori_op_sdpa, Dh = 64 on 16-bit operands): the caller's Q, V and
-// float key mask in the layouts attn32_kernel reads.  One block per (row, head) and
-// 64-key tile: Q rows pre-scaled by scale * log2(e) (rounded once more to T), the tile's
-// V rows transposed through LDS into V^T rows in vt_pos_bf16 key order (keys past seq_kv
-// zero), and the tile's 64-bit key-validity word (key < seq_kv and mask >= 0.5; the
-// mask is per batch row, so only head 0 writes it).
-template <typename T>
-__global__ __launch_bounds__(256) void sdpa_stage_kernel(const T* __restrict__ q, const T* __restrict__ v,
-                                                         const float* __restrict__ mask, int H, int Sq, int Skv,
-                                                         int vstride, float qmul, T* __restrict__ qs,
-                                                         T* __restrict__ vt, unsigned long long* __restrict__ bits) {
-    __shared__ T tile[64][64 + 2];
-    const int t = blockIdx.x, bh = blockIdx.y, b = bh / H, h = bh % H;
-    const int ntq = (Sq + 63) / 64, ntk = vstride / 64;
-    const int tid = threadIdx.x;
-    if (t < ntq) {  // 64 query rows of 64 dims
-        const size_t base = ((size_t)bh * Sq + (size_t)t * 64) * 64;
-        const int rows = Sq - t * 64 < 64 ? Sq - t * 64 : 64;
-        for (int i = tid; i < rows * 64; i += 256) qs[base + i] = static_cast<T>(static_cast<float>(q[base + i]) * qmul);
-    }
-    if (t >= ntk) return;
-    const int k0 = t * 64;
-    for (int i = tid; i < 64 * 64; i += 256) {
-        const int kk = i / 64, d = i % 64, key = k0 + kk;
-        tile[kk][d] = key < Skv ? v[((size_t)bh * Skv + key) * 64 + d] : static_cast<T>(0.f);
-    }
-    __syncthreads();
-    for (int i = tid; i < 64 * 64; i += 256) {
-        const int d = i / 64, kk = i % 64;
-        vt[((size_t)bh * 64 + d) * vstride + vt_pos_bf16(k0 + kk)] = tile[kk][d];
-    }
-    if (h == 0 && tid < 64) {
-        const int key = k0 + tid;
-        const bool ok = key < Skv && (mask == nullptr || mask[(size_t)b * Skv + key] >= 0.5f);
-        const unsigned long long w = __ballot(ok);
-        if (tid == 0) bits[(size_t)b * ntk + t] = w;
-    }
-}
-
 }  // namespace
 
 int launch_attention32(const AttnArgs<bf16>& a, hipStream_t st) { return launch_attention32_t<bf16>(a, st); }
-int launch_attention32(const AttnArgs<f16>& a, hipStream_t st) { return launch_attention32_t<f16>(a, st); }
-
-size_t sdpa_stage_bytes(int B, int H, int Sq, int Skv) {
-    const size_t vs = (size_t)(Skv + 63) / 64 * 64;
-    auto al = [](size_t n) { return (n + 255) / 256 * 256; };
-    return al((size_t)B * H * Sq * 64 * 2) + al((size_t)B * H * 64 * vs * 2) + al((size_t)B * (vs / 64) * 8);
-}
-
-template <typename T>
-int launch_sdpa_staged(const T* q, const T* k, const T* v, const float* mask, int B, int H, int Sq, int Skv,
-                       float scale, float* out, void* ws, size_t ws_bytes, hipStream_t st) {
-    const int vs = (Skv + 63) / 64 * 64;
-    if (B <= 0 || H <= 0 || Sq <= 0 || Skv <= 0 || vs / 64 > kAttnMaxKeyTiles) return -1;
-    if (ws_bytes < sdpa_stage_bytes(B, H, Sq, Skv) || ((uintptr_t)ws & 255)) return -1;
-    auto al = [](size_t n) { return (n + 255) / 256 * 256; };
-    unsigned char* p = static_cast<unsigned char*>(ws);
-    T* qs = reinterpret_cast<T*>(p);
-    T* vt = reinterpret_cast<T*>(p + al((size_t)B * H * Sq * 64 * 2));
-    unsigned long long* bits =
-        reinterpret_cast<unsigned long long*>(p + al((size_t)B * H * Sq * 64 * 2) + al((size_t)B * H * 64 * vs * 2));
-    const int ntq = (Sq + 63) / 64, ntk = vs / 64;
-    sdpa_stage_kernel<T><<<dim3(ntq > ntk ? ntq : ntk, B * H), 256, 0, st>>>(
-        q, v, mask, H, Sq, Skv, vs, scale * 1.4426950408889634f, qs, vt, bits);
-    AttnArgs<T> a{};
-    a.Q = qs;
-    a.K0 = k;
-    a.V0 = vt;
-    a.len0 = Skv;
-    a.stride0 = Skv;
-    a.bits0 = bits;
-    a.B = B;
-    a.H = H;
-    a.Sq = Sq;
-    a.scale = scale;
-    a.v_transposed = true;
-    a.prescaled = true;
-    a.vstride0 = vs;
-    a.out_mode = 1;
-    a.Of = out;
-    return launch_attention32_t<T>(a, st);
-}
-template int launch_sdpa_staged<bf16>(const bf16*, const bf16*, const bf16*, const float*, int, int, int, int, float,
-                                      float*, void*, size_t, hipStream_t);
-template int launch_sdpa_staged<f16>(const f16*, const f16*, const f16*, const float*, int, int, int, int, float,
-                                     float*, void*, size_t, hipStream_t);
 
 }  // namespace irodori

@@ -1,11 +1,9 @@
 // The SDPA operator entry points (native_fa_sdpa_wgsl / native_fa_sdpa_f16_in,
-// fused_sdpa_native.rs:220-302, fused_sdpa_native_f16.rs:181-200): argument checks, the
-// choice between the model's joint attention kernel (16-bit operands, head_dim 64, after
-// staging Q / V^T / key bits) and the generic flash kernel, and the staging buffer --
-// stream-ordered per call (irodori_op_sdpa) or a fixed per-GPU device array
-// (irodori_op_sdpa_noalloc, for callers that cannot allocate).
+// fused_sdpa_native.rs:220-302, fused_sdpa_native_f16.rs:181-200): argument checks and the
+// kernel by dtype -- 16-bit operands on the row-major flash kernel (kernels_attn_nv.hip), f32
+// on the generic one.  Neither needs device memory of its own, so irodori_op_sdpa and
+// irodori_op_sdpa_noalloc run the same launch; the latter keeps its contract's refusals.
 #include <atomic>
-#include <mutex>
 
 #include "../../include/irodori_hip.h"
 #include "common.hpp"
@@ -26,64 +24,46 @@ int check_sdpa_args(int dtype, const void* q, const void* k, const void* v, int 
     return IRODORI_OK;
 }
 
-// 16-bit operands with Dh = 64 run on the model's joint attention kernel after staging
-// (its tile list holds up to 16384 keys); everything else on the generic flash kernel.
-bool sdpa_staged(int dtype, int Dh, int Skv) {
-    return dtype != IRODORI_DTYPE_F32 && Dh == 64 && Skv <= 64 * kAttnMaxKeyTiles;
-}
-
 template <typename T>
-int sdpa_direct_t(const void* q, const void* k, const void* v, const float* mask, int B, int H, int Sq, int Skv, int Dh,
-                  float scale, float* out, hipStream_t st) {
+int sdpa_t(const void* q, const void* k, const void* v, const float* mask, int B, int H, int Sq, int Skv, int Dh,
+           float scale, float* out, hipStream_t st) {
     AttnArgs<T> a{};
     a.Q = static_cast<const T*>(q);
     a.K0 = static_cast<const T*>(k);
     a.V0 = static_cast<const T*>(v);
     a.len0 = Skv; a.stride0 = Skv; a.mask0 = mask;
     a.B = B; a.H = H; a.Sq = Sq; a.scale = scale; a.out_mode = 1; a.Of = out;
-    const int rc = Dh == 64 ? launch_attention<T, 64>(a, st) : launch_attention<T, 128>(a, st);
+    int rc;
+    if constexpr (sizeof(T) == 2)
+        rc = Dh == 64 ? launch_attention_nv<T, 64>(a, st) : launch_attention_nv<T, 128>(a, st);
+    else
+        rc = Dh == 64 ? launch_attention<T, 64>(a, st) : launch_attention<T, 128>(a, st);
     IRO_REQUIRE(rc == 0, IRODORI_ERR_SHAPE, "sdpa launch rejected the shape");
     return check_launch("sdpa");
 }
 
-int sdpa_direct(int dtype, const void* q, const void* k, const void* v, const float* mask, int B, int H, int Sq,
-                int Skv, int Dh, float scale, float* out, hipStream_t st) {
-    if (dtype == IRODORI_DTYPE_BF16) return sdpa_direct_t<bf16>(q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
-    if (dtype == IRODORI_DTYPE_F16) return sdpa_direct_t<f16>(q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
-    return sdpa_direct_t<float>(q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
+int sdpa_run(int dtype, const void* q, const void* k, const void* v, const float* mask, int B, int H, int Sq,
+             int Skv, int Dh, float scale, float* out, hipStream_t st) {
+    if (dtype == IRODORI_DTYPE_BF16) return sdpa_t<bf16>(q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
+    if (dtype == IRODORI_DTYPE_F16) return sdpa_t<f16>(q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
+    return sdpa_t<float>(q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
 }
 
-// The staged path on a caller-provided (or stream-ordered) buffer ws of `bytes`.
-int sdpa_run_staged(int dtype, const void* q, const void* k, const void* v, const float* mask, int B, int H, int Sq,
-                    int Skv, float scale, float* out, void* ws, size_t bytes, hipStream_t st) {
-    int rc;
-    if (dtype == IRODORI_DTYPE_BF16)
-        rc = launch_sdpa_staged<bf16>(static_cast<const bf16*>(q), static_cast<const bf16*>(k),
-                                      static_cast<const bf16*>(v), mask, B, H, Sq, Skv, scale, out, ws, bytes, st);
-    else
-        rc = launch_sdpa_staged<f16>(static_cast<const f16*>(q), static_cast<const f16*>(k),
-                                     static_cast<const f16*>(v), mask, B, H, Sq, Skv, scale, out, ws, bytes, st);
-    IRO_REQUIRE(rc == 0, IRODORI_ERR_SHAPE, "staged sdpa rejected the shape");
-    return check_launch("sdpa");
+// irodori_op_sdpa_noalloc's contract: 16-bit operands with Dh = 64 and at most 16384 keys are
+// held to IRODORI_SDPA_SCRATCH_BYTES of Q, V^T and key bits.
+bool noalloc_bounded(int dtype, int Dh, int Skv) { return dtype != IRODORI_DTYPE_F32 && Dh == 64 && Skv <= 16384; }
+size_t noalloc_bytes(int B, int H, int Sq, int Skv) {
+    const size_t vs = (size_t)(Skv + 63) / 64 * 64;
+    auto al = [](size_t n) { return (n + 255) / 256 * 256; };
+    return al((size_t)B * H * Sq * 64 * 2) + al((size_t)B * H * 64 * vs * 2) + al((size_t)B * (vs / 64) * 8);
 }
-
-// ---- fixed staging buffer of irodori_op_sdpa_noalloc ------------------------------------
-// One array per GPU the library runs on, held until the process ends.  In host code its
-// name is a host-side stand-in: kernels get the device address that hipGetSymbolAddress
-// returns for the current device, looked up once per device.
-static __device__ __align__(256) unsigned char scratch[IRODORI_SDPA_SCRATCH_BYTES];
 
 constexpr int kMaxDevices = 64;
-std::once_flag g_scratch_once[kMaxDevices];
-std::atomic<void*> g_scratch_ptr[kMaxDevices] = {};
-hipError_t g_scratch_rc[kMaxDevices] = {};
+std::atomic<bool> g_called[kMaxDevices] = {};
 
-// The scratch address on the device of `st`, which must be the current device (the address
-// is looked up with that device current, and the kernels run on the stream's device), or a
-// status code.  The lookup happens on the first call on a device; it is refused while `st`
-// is capturing (a first call inside a graph capture), so capturing callers make one eager
-// call first.
-int scratch_for_stream(hipStream_t st, void** out) {
+// The stream must be the current device's, and a device's first call (which loads the kernel's
+// code and sets its LDS limit) must not be captured: capturing callers make one eager call first.
+int check_noalloc_stream(hipStream_t st) {
     int dev = -1;
     IRO_HIP_CHECK(hipGetDevice(&dev));
     if (st) {
@@ -93,25 +73,15 @@ int scratch_for_stream(hipStream_t st, void** out) {
                     "irodori_op_sdpa_noalloc: the stream belongs to device " + std::to_string(sdev) +
                         " but device " + std::to_string(dev) + " is current; make the stream's device current");
     }
-    IRO_REQUIRE(dev >= 0 && dev < kMaxDevices, IRODORI_ERR_INVALID_ARG, "device index beyond the scratch table");
-    if (!g_scratch_ptr[dev].load()) {
+    IRO_REQUIRE(dev >= 0 && dev < kMaxDevices, IRODORI_ERR_INVALID_ARG, "device index beyond the device table");
+    if (!g_called[dev].load()) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         IRO_HIP_CHECK(hipStreamIsCapturing(st, &cs));
         IRO_REQUIRE(cs == hipStreamCaptureStatusNone, IRODORI_ERR_INVALID_ARG,
-                    "irodori_op_sdpa_noalloc: the first call on a device must not be under graph capture "
-                    "(it looks up the fixed buffer's address); make one call outside the capture first");
+                    "irodori_op_sdpa_noalloc: the first call on a device must not be under graph capture; make "
+                    "one call outside the capture first");
+        g_called[dev].store(true);
     }
-    std::call_once(g_scratch_once[dev], [dev] {
-        void* p = nullptr;
-        g_scratch_rc[dev] = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        g_scratch_ptr[dev].store(p);
-    });
-    void* p = g_scratch_ptr[dev].load();
-    if (g_scratch_rc[dev] != hipSuccess || !p) {
-        set_last_error(std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(g_scratch_rc[dev]));
-        return IRODORI_ERR_HIP;
-    }
-    *out = p;
     return IRODORI_OK;
 }
 
@@ -123,17 +93,7 @@ int irodori_op_sdpa(int dtype, const void* q, const void* k, const void* v, cons
                     int Skv, int Dh, float scale, float* out, void* stream) {
     IRO_GUARD_BEGIN
     IRO_TRY(check_sdpa_args(dtype, q, k, v, B, H, Sq, Skv, Dh, out));
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    if (!sdpa_staged(dtype, Dh, Skv)) return sdpa_direct(dtype, q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
-    // Staging buffer in stream order: overlapping calls on different streams never share it.
-    const size_t bytes = sdpa_stage_bytes(B, H, Sq, Skv);
-    void* ws = nullptr;
-    IRO_HIP_CHECK(hipMallocAsync(&ws, bytes, st));
-    const int rc = sdpa_run_staged(dtype, q, k, v, mask, B, H, Sq, Skv, scale, out, ws, bytes, st);
-    const hipError_t fe = hipFreeAsync(ws, st);
-    if (rc != IRODORI_OK) return rc;
-    IRO_HIP_CHECK(fe);
-    return IRODORI_OK;
+    return sdpa_run(dtype, q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, static_cast<hipStream_t>(stream));
     IRO_GUARD_END
 }
 
@@ -142,17 +102,15 @@ int irodori_op_sdpa_noalloc(int dtype, const void* q, const void* k, const void*
     IRO_GUARD_BEGIN
     IRO_TRY(check_sdpa_args(dtype, q, k, v, B, H, Sq, Skv, Dh, out));
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (!sdpa_staged(dtype, Dh, Skv)) return sdpa_direct(dtype, q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
-    const size_t bytes = sdpa_stage_bytes(B, H, Sq, Skv);
-    IRO_REQUIRE(bytes <= IRODORI_SDPA_SCRATCH_BYTES, IRODORI_ERR_SHAPE,
-                "irodori_op_sdpa_noalloc: the staging of this shape takes " + std::to_string(bytes) +
-                    " bytes, above the fixed " + std::to_string((size_t)IRODORI_SDPA_SCRATCH_BYTES) +
-                    "-byte buffer; use irodori_op_sdpa");
-    void* ws = nullptr;
-    IRO_TRY(scratch_for_stream(st, &ws));
-    // The staging kernel writes every byte the attention kernel reads (Q rows, V^T with zero
-    // keys past seq_kv, the key bits), so nothing left by an earlier call is read.
-    return sdpa_run_staged(dtype, q, k, v, mask, B, H, Sq, Skv, scale, out, ws, IRODORI_SDPA_SCRATCH_BYTES, st);
+    if (noalloc_bounded(dtype, Dh, Skv)) {
+        const size_t bytes = noalloc_bytes(B, H, Sq, Skv);
+        IRO_REQUIRE(bytes <= IRODORI_SDPA_SCRATCH_BYTES, IRODORI_ERR_SHAPE,
+                    "irodori_op_sdpa_noalloc: the operands of this shape take " + std::to_string(bytes) +
+                        " bytes, above the entry point's " + std::to_string((size_t)IRODORI_SDPA_SCRATCH_BYTES) +
+                        "; use irodori_op_sdpa");
+        IRO_TRY(check_noalloc_stream(st));
+    }
+    return sdpa_run(dtype, q, k, v, mask, B, H, Sq, Skv, Dh, scale, out, st);
     IRO_GUARD_END
 }
 

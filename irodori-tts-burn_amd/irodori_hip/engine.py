@@ -561,7 +561,7 @@ class ops:
     @staticmethod
     def sdpa_noalloc(dtype: int, d_q, d_k, d_v, d_mask, batch, heads, seq_q, seq_kv, head_dim, scale,
                      d_out, stream: int = 0) -> None:
-        """sdpa without any device allocation: the staging lives in the library's fixed
-        per-GPU buffer (SDPA_SCRATCH_BYTES); overlapping calls on one GPU race."""
+        """sdpa for callers that cannot allocate device memory: the same kernels and results, 16-bit
+        64-dim operands limited to SDPA_SCRATCH_BYTES, the first call on a GPU outside capture."""
         _check(L.load().irodori_op_sdpa_noalloc(dtype, d_q, d_k, d_v, d_mask or None, batch, heads, seq_q,
                                                 seq_kv, head_dim, scale, d_out, stream or None))

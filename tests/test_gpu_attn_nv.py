@@ -1,0 +1,59 @@
+"""The 16-bit SDPA operator on row-major K / V (kernels_attn_nv.hip) against the float64 oracle,
+at the edges of its tiles, key parities, tile words and workgroup shapes.
+
+Tolerance: the scores and sums are f32, so the error is the rounding of the probabilities to the
+operand dtype, at most half a unit in the last place of each (2^-9 in bf16, 2^-12 in f16) on
+terms of random sign: the relative L2 stays below twice that."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import rel_l2
+from irodori_hip import _lib as L
+from irodori_hip.engine import ops
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"bf16": (L.DTYPE_BF16, torch.bfloat16, 2.0 ** -8), "f16": (L.DTYPE_F16, torch.float16, 2.0 ** -11)}
+# B, H, Sq, Skv, Dh, mask, scale / Dh^-1/2.  Masks: None, "tail" (ragged rows), "holes" (whole
+# tiles and single keys dropped), "none valid" in the last row.
+CASES = [
+    (1, 1, 1, 1, 64, None, 1.0), (1, 2, 33, 65, 64, None, 1.0), (2, 3, 64, 128, 64, "tail", 1.0),
+    (3, 2, 65, 129, 64, "holes", 1.0), (1, 2, 40, 4100, 64, "holes", 1.0), (2, 2, 37, 200, 64, "empty", 1.0),
+    (1, 1, 1, 1, 128, None, 1.0), (1, 2, 31, 64, 128, "tail", 1.0), (2, 3, 65, 193, 128, "holes", 1.0),
+    (1, 2, 40, 4161, 128, "holes", 1.0), (2, 2, 37, 200, 128, "empty", 1.0),
+    (2, 16, 641, 70, 128, "tail", 1.0),                               # four query blocks per workgroup
+    (1, 2, 50, 150, 64, "tail", -3.0), (1, 2, 50, 150, 128, "tail", 0.0), (1, 2, 50, 150, 64, "holes", 40.0),
+]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("B,H,Sq,Skv,Dh,mask,mul", CASES)
+def test_row_major_attention(oracle64, dtype, B, H, Sq, Skv, Dh, mask, mul):
+    code, tdt, tol = TYPES[dtype]
+    rng = np.random.default_rng(Sq * 7 + Skv)
+    dq, dk, dv = (torch.from_numpy(rng.standard_normal((B, H, n, Dh)).astype(np.float32)).to("cuda").to(tdt)
+                  for n in (Sq, Skv, Skv))
+    m = np.ones((B, Skv), np.float32)
+    if mask == "tail":
+        for b in range(B):
+            m[b, max(1, Skv - 1 - 67 * b):] = 0
+    elif mask == "holes":
+        m[:, 64:min(Skv, 4000):3] = 0
+        m[0, 70:max(71, Skv - 66)] = 0
+    elif mask == "empty":
+        m[-1] = 0
+    out = torch.full((B, H, Sq, Dh), 7.0, dtype=torch.float32, device="cuda")
+    scale = mul * Dh ** -0.5
+    dm = torch.from_numpy(m).to("cuda")
+    ops.sdpa(code, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), 0 if mask is None else dm.data_ptr(), B, H, Sq, Skv,
+             Dh, scale, out.data_ptr())
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    want = oracle64.sdpa(*(a.float().cpu().numpy() for a in (dq, dk, dv)), m, scale)
+    assert np.isfinite(got).all()
+    if mask == "empty":
+        assert not got[-1].any()
+    err = rel_l2(got, want)
+    print("%s %s: rel L2 %.2e" % (dtype, (B, H, Sq, Skv, Dh, mask, mul), err))
+    assert err < tol

@@ -210,6 +210,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
     constexpr int BK = 128 / ES;                  // elements per slice
     constexpr int KS = BK / (F8 ? 64 : 16);       // MFMA k-steps per slice
     static_assert(!F8 || sizeof(T) == 2, "fp8 operands produce bf16 / f32 outputs");
+    static_assert(KS % 2 == 0, "a slice's first step reads fragment set 0");
     static_assert(LPW * 8 * NW == ROWS, "rows per slice must split over the waves");
     static_assert(FM * 32 == WM && FN * 32 == WN, "wave tiles are whole 32x32 blocks");
     static_assert(BM % 8 == 0, "a load instruction covers A rows or W rows, not both");
@@ -254,11 +255,15 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
     const unsigned char* Ab = F8 ? a.A8 : reinterpret_cast<const unsigned char*>(a.A);
     const unsigned char* Wb = F8 ? a.W8 : reinterpret_cast<const unsigned char*>(a.W);
     const __amdgpu_buffer_rsrc_t rA = make_rsrc(Ab + (size_t)m0 * lda * ES, (unsigned)((size_t)arows * lda * ES));
-    const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wb + (size_t)n0 * K * ES, (unsigned)(BN * K * ES));
     // W row rr of the tile: group rr / 64 at 64 K ES bytes in either layout; within the
     // group rows are K ES bytes apart (row-major) or 128 (tile-major, where consecutive
-    // slices are 8 KB apart instead of 128 bytes).
+    // slices are 8 KB apart instead of 128 bytes).  A 32-wide tile is one half of a group.
     const bool wt = !CONV && a.w_tiled;
+    constexpr int BN64 = BN < 64 ? 64 : BN;
+    const int ng = n0 / BN64 * BN64;
+    const size_t w_bytes = (size_t)BN64 * K * ES;
+    const size_t w_skip = (size_t)(n0 - ng) * (wt ? 128 : (size_t)K * ES);
+    const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wb + (size_t)ng * K * ES + w_skip, (unsigned)(w_bytes - w_skip));
     const unsigned w_row = wt ? 128u : (unsigned)(K * ES), w_slice = wt ? 8192u : 128u;
     unsigned voff[LPW];
 #pragma unroll
@@ -297,23 +302,25 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
         }
         __syncthreads();
     }
-#define GEMM_ISSUE(kt_, stage_)                                                            \
-    do {                                                                                   \
-        unsigned char* dst_ = smem + (stage_) * STAGE_BYTES + wave * LPW * 1024;           \
-        const unsigned ws_ = (unsigned)(kt_) * w_slice;                                    \
-        unsigned as_ = (unsigned)(kt_) * 128u;                                             \
-        bool split_ = false;                                                               \
-        if constexpr (CONV) {                                                              \
-            const int k0_ = (kt_) * BK, j0_ = k0_ / a.conv_cp;                             \
-            as_ += (unsigned)j0_ * conv_dstep;                                             \
-            split_ = k0_ - j0_ * a.conv_cp + BK > a.conv_cp;                               \
-        }                                                                                  \
-        _Pragma("unroll") for (int i_ = 0; i_ < LPW; i_++) {                               \
-            const bool isA = (wave * LPW + i_) * 8 < BM;                                   \
-            const unsigned vo_ = (CONV && isA && split_) ? voff_hi[i_] : voff[i_];         \
-            buf_load_lds16(isA ? rA : rW, vo_, isA ? as_ : ws_, dst_ + i_ * 1024);         \
-        }                                                                                  \
-    } while (0)
+    // Load instructions [i0_, i1_) of this wave for slice kt_ into its ring stage.
+    auto issue = [&](int kt, int stage, int i0, int i1) {
+        unsigned char* dst = smem + stage * STAGE_BYTES + wave * LPW * 1024;
+        const unsigned ws = (unsigned)kt * w_slice;
+        unsigned as = (unsigned)kt * 128u;
+        bool split = false;
+        if constexpr (CONV) {
+            const int k0 = kt * BK, j0 = k0 / a.conv_cp;
+            as += (unsigned)j0 * conv_dstep;
+            split = k0 - j0 * a.conv_cp + BK > a.conv_cp;
+        }
+#pragma unroll
+        for (int i = 0; i < LPW; i++) {
+            if (i < i0 || i >= i1) continue;
+            const bool isA = (wave * LPW + i) * 8 < BM;
+            const unsigned vo = (CONV && isA && split) ? voff_hi[i] : voff[i];
+            buf_load_lds16(isA ? rA : rW, vo, isA ? as : ws, dst + i * 1024);
+        }
+    };
 
     f32x16 acc[FM][FN];
 #pragma unroll
@@ -435,100 +442,150 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
             sq = sq >= a.S ? sq - a.S : sq;
         }
     };
+    // Main loop.  The fragments of step ks + 1 are read ahead of the MFMAs of step ks.  With three
+    // stages or more (PIPE) the loop is pipelined over the slices too: the next slice's first
+    // fragments are read ahead of the MFMAs of this slice's last step, after the barrier that
+    // makes that slice visible, and the loads of slice kt + STAGES - 1 go out in parts between
+    // the MFMAs of slice kt's earlier steps.  A slice of a 64x64 tile (4 MFMAs a wave) takes 0.16
+    // instead of 0.26 us that way, one of a 128x128 tile 0.35 instead of 0.45 (W2 750 x 2816 x
+    // 1024: 15.8 -> 12.4 us).  With two stages the wait for the only slice in flight must come as
+    // late as possible, at the start of its own slice (pipelined, the 750-frame RF run took 47.8
+    // instead of 45.5 ms).
+    constexpr bool PIPE = STAGES > 2;
 #pragma unroll
     for (int s = 0; s < STAGES - 1; s++)
-        if (s < nk) GEMM_ISSUE(s, s);
+        if (s < nk) issue(s, s, 0, LPW);
     const int fr = lane & 31, fh = lane >> 5;
-    for (int kt = 0; kt < nk; kt++) {
-        // Slice kt has landed (the min(STAGES - 2, nk - 1 - kt) slices issued after it may
-        // still be in flight); make it visible.
-        wait_slices<STAGES - 2, LPW>(nk - 1 - kt);
-        raw_barrier();
-        if (kt + STAGES - 1 < nk) GEMM_ISSUE(kt + STAGES - 1, (kt + STAGES - 1) % STAGES);
-        if constexpr (EPI == EPI_QKVG) {
-            // The stage after the last slice's was last read in iteration nk - 2, which every
-            // wave has finished at this barrier: the RoPE rows of the tile stream into it
-            // while the last slice's MFMAs run.
-            if (rope_wg && kt == nk - 1) rope_rows_issue(smem + (nk % STAGES) * STAGE_BYTES);
-        }
-        if constexpr (FUSE_IN) {
-            if (a.rstat && kt == 0) {
+    using FragT = typename std::conditional<F8, Frag8, Frag32<T>>::type;
+    FragT af[2][FM], bfr[2][FN];
+    [[maybe_unused]] unsigned scw[FM], scn[FM];  // fp8: scale bytes of this lane's rows, this and the next slice
+    auto read_step = [&](int stage, int ks, int set) {
+        const unsigned char* st = smem + stage * STAGE_BYTES;
 #pragma unroll
-                for (int p = 0; p < RPL; p++) {
-                    float ss = 0.f;
-#pragma unroll
-                    for (int q = 0; q < 16; q++) {
-                        ss += rsv[p][q].x;
-                        ss += rsv[p][q].y;
-                        ss += rsv[p][q].z;
-                        ss += rsv[p][q].w;
-                    }
-                    rown[p] = m0 + wm0 + 64 * p + lane < a.M ? 1.f / sqrtf(ss / (float)K + a.eps) : 1.f;
-                }
-            }
+        for (int i = 0; i < FM; i++) {
+            if constexpr (F8) af[set][i] = read_frag8(st, wm0 + 32 * i + fr, ks, fh);
+            else af[set][i] = read_frag<T>(st, wm0 + 32 * i + fr, ks, fh);
         }
-        const unsigned char* st = smem + (kt % STAGES) * STAGE_BYTES;
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            if constexpr (F8) bfr[set][j] = read_frag8(st, BM + wn0 + 32 * j + fr, ks, fh);
+            else bfr[set][j] = read_frag<T>(st, BM + wn0 + 32 * j + fr, ks, fh);
+        }
+    };
+    auto read_scales = [&](int kt) {
         if constexpr (F8) {
-            // Scale bytes of this lane's rows for the slice's four k blocks.
-            unsigned scw[FM];
-#pragma unroll
-            for (int i = 0; i < FM; i++) scw[i] = *reinterpret_cast<const unsigned*>(sc_lds + (kt * BM + wm0 + 32 * i + fr) * 4);
-            // Fragments double-buffered as in the bf16 loop: the reads of step ks + 1 go out
-            // ahead of the MFMAs of step ks (two 16-byte LDS reads per fragment).
-            Frag8 af8[2][FM], bf8[2][FN];
-#pragma unroll
-            for (int i = 0; i < FM; i++) af8[0][i] = read_frag8(st, wm0 + 32 * i + fr, 0, fh);
-#pragma unroll
-            for (int j = 0; j < FN; j++) bf8[0][j] = read_frag8(st, BM + wn0 + 32 * j + fr, 0, fh);
-            __builtin_amdgcn_sched_group_barrier(0x100, 2 * (FM + FN), 0);
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const int cur = ks & 1, nxt = cur ^ 1;
-                if (ks + 1 < KS) {
-#pragma unroll
-                    for (int i = 0; i < FM; i++) af8[nxt][i] = read_frag8(st, wm0 + 32 * i + fr, ks + 1, fh);
-#pragma unroll
-                    for (int j = 0; j < FN; j++) bf8[nxt][j] = read_frag8(st, BM + wn0 + 32 * j + fr, ks + 1, fh);
-                }
-#pragma unroll
-                for (int i = 0; i < FM; i++) {
-                    const int sa = (int)((scw[i] >> (8 * (2 * ks + fh))) & 0xffu);
-#pragma unroll
-                    for (int j = 0; j < FN; j++) mma8(acc[i][j], af8[cur][i], bf8[cur][j], sa);
-                }
-                if (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, 2 * (FM + FN), 0);  // DS reads
-                __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);                         // MFMAs
-            }
-            continue;
-        }
-        // Fragments double-buffered in registers: the LDS reads of k16 step ks + 1 are
-        // issued ahead of the MFMAs of step ks, so their latency hides behind FM*FN MFMAs.
-        Frag32<T> af[2][FM], bfr[2][FN];
-#pragma unroll
-        for (int i = 0; i < FM; i++) af[0][i] = read_frag<T>(st, wm0 + 32 * i + fr, 0, fh);
-#pragma unroll
-        for (int j = 0; j < FN; j++) bfr[0][j] = read_frag<T>(st, BM + wn0 + 32 * j + fr, 0, fh);
-        if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const int cur = ks & 1, nxt = cur ^ 1;
-            if (ks + 1 < KS) {
-#pragma unroll
-                for (int i = 0; i < FM; i++) af[nxt][i] = read_frag<T>(st, wm0 + 32 * i + fr, ks + 1, fh);
-#pragma unroll
-                for (int j = 0; j < FN; j++) bfr[nxt][j] = read_frag<T>(st, BM + wn0 + 32 * j + fr, ks + 1, fh);
-            }
 #pragma unroll
             for (int i = 0; i < FM; i++)
+                scn[i] = *reinterpret_cast<const unsigned*>(sc_lds + (kt * BM + wm0 + 32 * i + fr) * 4);
+        }
+    };
+    if constexpr (FUSE_IN) {
+        // Row scales, while the first slices are in flight.
+        if (a.rstat) {
 #pragma unroll
-                for (int j = 0; j < FN; j++) mma32(acc[i][j], af[cur][i], bfr[cur][j]);
-            if constexpr (sizeof(T) == 2) {
-                if (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);  // DS reads
-                __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);                   // MFMAs
+            for (int p = 0; p < RPL; p++) {
+                float ss = 0.f;
+#pragma unroll
+                for (int q = 0; q < 16; q++) {
+                    ss += rsv[p][q].x;
+                    ss += rsv[p][q].y;
+                    ss += rsv[p][q].z;
+                    ss += rsv[p][q].w;
+                }
+                rown[p] = m0 + wm0 + 64 * p + lane < a.M ? 1.f / sqrtf(ss / (float)K + a.eps) : 1.f;
             }
         }
     }
-#undef GEMM_ISSUE
+    int st = 0;  // ring stage of slice kt
+    if constexpr (PIPE) {
+        wait_slices<STAGES - 2, LPW>(nk - 1);
+        raw_barrier();
+        read_step(0, 0, 0);
+        read_scales(0);
+    }
+    auto mma_step = [&](int ks) {
+#pragma unroll
+        for (int i = 0; i < FM; i++) {
+            if constexpr (F8) {
+                const int sa = (int)((scw[i] >> (8 * (2 * ks + fh))) & 0xffu);
+#pragma unroll
+                for (int j = 0; j < FN; j++) mma8(acc[i][j], af[ks & 1][i], bfr[ks & 1][j], sa);
+            } else {
+#pragma unroll
+                for (int j = 0; j < FN; j++) mma32(acc[i][j], af[ks & 1][i], bfr[ks & 1][j]);
+            }
+        }
+    };
+    // PIPE: loads issued before step ks of a slice.
+    auto part = [](int ks) { return ks * LPW / (KS - 1); };
+    constexpr int RD = (F8 ? 2 : 1) * (FM + FN);  // LDS reads of a step
+    // MORE: slice kt + STAGES - 1 is loaded during this one; LAST: the last slice.  During the
+    // last slice the tile's RoPE rows (QKVG) stream into the stage after it, which was last read
+    // in slice nk - 2: every wave is past that.
+    auto slice = [&](auto more_c, auto last_c, int kt) {
+        constexpr bool MORE = decltype(more_c)::value, LAST = decltype(last_c)::value;
+        const int stn = st + 1 == STAGES ? 0 : st + 1, stl = st == 0 ? STAGES - 1 : st - 1;
+        if constexpr (!PIPE) {
+            wait_vmcnt<0>();
+            raw_barrier();
+            if constexpr (MORE) issue(kt + 1, stl, 0, LPW);
+            if constexpr (LAST && EPI == EPI_QKVG) {
+                if (rope_wg) rope_rows_issue(smem + (nk % STAGES) * STAGE_BYTES);
+            }
+            read_scales(kt);
+            read_step(st, 0, 0);
+            if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_group_barrier(0x100, RD, 0);
+        }
+        if constexpr (F8) {
+#pragma unroll
+            for (int i = 0; i < FM; i++) scw[i] = scn[i];
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks + 1 < KS) {
+                read_step(st, ks + 1, (ks + 1) & 1);
+                if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (PIPE && MORE) issue(kt + STAGES - 1, stl, part(ks), part(ks + 1));
+            } else if constexpr (PIPE && !LAST) {
+                // Slice kt + 1 has landed (the min(STAGES - 2, nk - 2 - kt) slices issued after
+                // it may still be in flight) and this wave has read all of slice kt, whose
+                // stage is refilled after the barrier.
+                if constexpr (MORE) wait_slices<STAGES - 2, LPW>(STAGES - 2);
+                else wait_slices<STAGES - 2, LPW>(nk - 2 - kt);
+                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+                raw_barrier();
+                read_step(stn, 0, 0);
+                read_scales(kt + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            mma_step(ks);
+            if constexpr (!PIPE) {
+                if constexpr (sizeof(T) == 2) {
+                    if (ks + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, RD, 0);  // DS reads
+                    __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);              // MFMAs
+                }
+                continue;
+            }
+            if (MORE && ks + 1 < KS) {
+                // The step's loads between its MFMAs.
+                const int nl = part(ks + 1) - part(ks);
+#pragma unroll
+                for (int q = 0; q < (FM * FN > nl ? FM * FN : nl); q++) {
+                    if (q < FM * FN) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    if (q < nl) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        st = stn;
+    };
+    int kt = 0;
+    for (; kt < nk - (STAGES - 1); kt++) slice(std::true_type{}, std::false_type{}, kt);
+    for (; kt < nk - 1; kt++) slice(std::false_type{}, std::false_type{}, kt);
+    if constexpr (EPI == EPI_QKVG && PIPE) {
+        if (rope_wg) rope_rows_issue(smem + (nk % STAGES) * STAGE_BYTES);
+    }
+    slice(std::false_type{}, std::true_type{}, kt);
 
     if constexpr (F8) {  // per-output-channel weight scales
 #pragma unroll
@@ -1300,7 +1357,8 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
                  a.next_layer >= a.mt.layers || a.next_kind < 0 || a.next_kind > 1))
         return -1;
     if ((size_t)BN * a.K * ES > 0xffffffffull || (size_t)BM * a.K * ES > 0xffffffffull) return -1;
-    if (a.w_tiled && (CONV || BN % 64 != 0)) return -1;
+    if (a.w_tiled && (CONV || (BN % 64 != 0 && BN != 32) || a.N % 64 != 0)) return -1;
+    if (BN < 64 && a.N % 64 != 0) return -1;  // the weight resource spans whole 64-row groups
     if (CONV) {
         // conv_cp a multiple of half a slice (a slice straddles at most two taps, at its
         // middle); K = the taps' span rounded up to whole slices.
@@ -1346,19 +1404,44 @@ void launch_tile_rows(const void* src, int N, int row_bytes, void* dst, hipStrea
                                                                         static_cast<unsigned char*>(dst));
 }
 
-// Tile choice per epilogue.  With 2x2 wavefronts of 32x32 blocks the main loop is bound by
-// LDS bandwidth (fragment reads + the DMA writes): 1.5x the MFMA time for 128x128 tiles,
-// 3x for 64x64.  The wide projections (QKV+gate, W1|W3) use 128x128 tiles in two stages
-// (two workgroups per CU); the D-wide projections (Wo, W2) use 64x64 tiles in four stages
-// so that N = 1024 still yields enough workgroups (split-K over larger tiles measured
-// slower: the f32 partial planes cost more HBM traffic than the LDS time they save), unless
-// the batch is large enough for 128x128 tiles.
-// Large batches (many utterances) fill the chip with 128x128 tiles too: two full waves of
-// workgroups (two per CU) or more.  Tiles are the same MFMA sequence over k in either
-// shape, so the choice does not change a single output bit.
+// Tile choice per epilogue.  A tile's per-output arithmetic is the same MFMA sequence over k in
+// every shape, so no choice changes an output bit.  What differs is how many workgroups a launch
+// has for the 256 CUs and how much of its time is the chain of slices in each:
+//   * Large launches: 128x128 tiles in two stages, two workgroups per CU; with 2x2 wavefronts
+//     of 32x32 blocks the LDS traffic is 1.5x the MFMA time (3x for 64x64).
+//   * Launches that leave CUs idle at that size (one utterance's rows at N = 4 D or 2 F) take
+//     smaller tiles in three or four stages with the pipelined loop, more workgroups and
+//     shorter slices.  8 steps of the d1024 sampler, ms, with QKV+gate tiles / W1|W3 tiles of
+//     128x128 -> the choice below: 24 frames 8.30 -> 7.08, 128 frames 8.14 -> 6.01, 256 frames 7.92 ->
+//     6.49, 384 frames 8.14 -> 7.06, 512 frames 8.29 -> 7.90, 640 frames 8.89 -> 8.60; at 750 and beyond
+//     128x128 is the better one (40 steps 45.5 against 45.8 and 47.0 ms).
+//   * The D-wide residual projections: 64x64 in four stages, 32x64 while that still leaves most
+//     CUs one workgroup at most (8 steps at 128 frames 7.79 -> 7.44, 384 frames 8.14 -> 7.80, 512 frames 8.29 ->
+//     8.55), 128x128 for batches that give two workgroups per CU.
 template <typename T>
 static bool wide_enough(const GemmArgs<T>& a) {
     return a.N % 128 == 0 && (long)((a.M + 127) / 128) * (a.N / 128) >= 512;
+}
+static long tile_count(int M, int N, int bm, int bn) { return (long)((M + bm - 1) / bm) * (N / bn); }
+
+// QKV+gate with 64-dim heads (one head per wave).
+template <typename T, bool F8>
+static int launch_qkvg(const GemmArgs<T>& a, hipStream_t st) {
+    if (tile_count(a.M, a.N, 64, 64) <= 256) return launch_cfg<T, 64, 64, 2, 1, 4, EPI_QKVG, F8>(a, st);
+    if (tile_count(a.M, a.N, 64, 128) <= 320) return launch_cfg<T, 64, 128, 2, 2, 3, EPI_QKVG, F8>(a, st);
+    return launch_cfg<T, 128, 128, 2, 2, 2, EPI_QKVG, F8>(a, st);
+}
+template <typename T, bool F8>
+static int launch_swiglu(const GemmArgs<T>& a, hipStream_t st) {
+    if (tile_count(a.M, a.N, 64, 64) <= 256) return launch_cfg<T, 64, 64, 2, 1, 4, EPI_SWIGLU, F8>(a, st);
+    if (tile_count(a.M, a.N, 128, 64) <= 352) return launch_cfg<T, 128, 64, 4, 1, 3, EPI_SWIGLU, F8>(a, st);
+    return launch_cfg<T, 128, 128, 2, 2, 2, EPI_SWIGLU, F8>(a, st);
+}
+template <typename T, bool F8>
+static int launch_resid(const GemmArgs<T>& a, hipStream_t st) {
+    if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_RESID, F8>(a, st);
+    if (tile_count(a.M, a.N, 32, 64) <= 192) return launch_cfg<T, 32, 64, 1, 2, 5, EPI_RESID, F8>(a, st);
+    return launch_cfg<T, 64, 64, 2, 2, 4, EPI_RESID, F8>(a, st);
 }
 
 template <typename T>
@@ -1369,18 +1452,17 @@ int launch_gemm(int epi, const GemmArgs<T>& a, hipStream_t st) {
             if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_STORE>(a, st);
             return launch_cfg<T, 64, 64, 2, 2, 4, EPI_STORE>(a, st);
         case EPI_RESID:
-            if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_RESID>(a, st);
-            return launch_cfg<T, 64, 64, 2, 2, 4, EPI_RESID>(a, st);
+            return launch_resid<T, false>(a, st);
         case EPI_ADD:
             if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_ADD>(a, st);
             if (a.N % 128 != 0 && a.N % 192 == 0 && (long)((a.M + 127) / 128) * (a.N / 192) >= 512)
                 return launch_cfg<T, 128, 192, 2, 2, 2, EPI_ADD>(a, st);
             return launch_cfg<T, 64, 64, 2, 2, 4, EPI_ADD>(a, st);
-        case EPI_SWIGLU: return launch_cfg<T, 128, 128, 2, 2, 2, EPI_SWIGLU>(a, st);
+        case EPI_SWIGLU: return launch_swiglu<T, false>(a, st);
         // QKVG / CTXKV: one head per wave, 2 x 2 waves of 64 columns or 4 x 1 of 128.
         case EPI_QKVG:
             if (a.H > 0 && a.D == a.H * 128) return launch_cfg<T, 128, 128, 4, 1, 2, EPI_QKVG>(a, st);
-            return launch_cfg<T, 128, 128, 2, 2, 2, EPI_QKVG>(a, st);
+            return launch_qkvg<T, false>(a, st);
         case EPI_CTXKV:
             if (a.H > 0 && a.D == a.H * 128) return launch_cfg<T, 128, 128, 4, 1, 2, EPI_CTXKV>(a, st);
             return launch_cfg<T, 128, 128, 2, 2, 2, EPI_CTXKV>(a, st);
@@ -1396,10 +1478,9 @@ int launch_gemm_fp8(int epi, const GemmArgs<bf16>& a, hipStream_t st) {
             if (wide_enough(a)) return launch_cfg<bf16, 128, 128, 2, 2, 2, EPI_STORE, true>(a, st);
             return launch_cfg<bf16, 64, 64, 2, 2, 4, EPI_STORE, true>(a, st);
         case EPI_RESID:
-            if (wide_enough(a)) return launch_cfg<bf16, 128, 128, 2, 2, 2, EPI_RESID, true>(a, st);
-            return launch_cfg<bf16, 64, 64, 2, 2, 4, EPI_RESID, true>(a, st);
-        case EPI_SWIGLU: return launch_cfg<bf16, 128, 128, 2, 2, 2, EPI_SWIGLU, true>(a, st);
-        case EPI_QKVG: return launch_cfg<bf16, 128, 128, 2, 2, 2, EPI_QKVG, true>(a, st);
+            return launch_resid<bf16, true>(a, st);
+        case EPI_SWIGLU: return launch_swiglu<bf16, true>(a, st);
+        case EPI_QKVG: return launch_qkvg<bf16, true>(a, st);
     }
     return -1;
 }

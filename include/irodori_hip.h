@@ -271,10 +271,7 @@ int irodori_op_joint_attention(irodori_ctx* ctx, int layer, int batch, int seq, 
  * x += gate * SwiGlu(x / rms(x) * (1 + scale) + shift) (norm.rs:160-169,
  * feed_forward.rs:76-85), with the caller's modulation vectors shift / scale / gate
  * [batch, D] f32 (gate as applied, after tanh) and the context's norm_eps; x [batch, seq, D]
- * f32, updated in place.  bf16 contexts with the fused adaLN run each row as a sampler
- * chain does (the norm folded into the W1|W3 GEMM); otherwise the adaLN kernel, W1|W3 and W2
- * over all rows.  Overwrites the context's modulation table rows 0..batch-1 of (layer,
- * mlp), which the next forward or sampling call rebuilds. */
+ * f32, updated in place.  The adaLN kernel, W1|W3 and W2 over all rows. */
 int irodori_op_swiglu_mlp(irodori_ctx* ctx, int layer, int batch, int seq, float* x,
                           const float* shift, const float* scale, const float* gate, void* stream);
 

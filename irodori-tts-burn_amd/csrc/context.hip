@@ -441,6 +441,7 @@ enum LayerPart {
 struct PartOpts {
     float* x = nullptr;
     bool no_next = false;
+    bool unfused = false;  // the adaLN kernel whatever mt would allow (an isolated MLP half)
 };
 
 // One kernel of a DiT block over batch rows [r0, r0 + B) of the context's buffers, on
@@ -467,7 +468,7 @@ int enqueue_part(irodori_ctx* c, int l, int B, int S, const ModTable& mt, int pa
     // fp8 compute: the e4m3 copies of h / o / u with their block scales (same row slice).
     const bool f8 = c->fp8 && std::is_same<T, bf16>::value;
     // Fused adaLN (bf16): the partial sums of the slice's rows and this layer's shift biases.
-    const bool fz = std::is_same<T, bf16>::value && fused_for(c, mt, B);
+    const bool fz = std::is_same<T, bf16>::value && !opt.unfused && fused_for(c, mt, B);
     float* rstat = fz ? c->rstat + tok0 * (D / 32) : nullptr;
     uint8_t* h8 = f8 ? c->h8 + tok0 * D : nullptr;
     uint8_t* h8s = f8 ? c->h8s + tok0 * (D / 32) : nullptr;
@@ -1862,51 +1863,24 @@ int irodori_op_swiglu_mlp(irodori_ctx* c, int layer, int B, int S, float* x, con
                 "batch must be in [1, max_rows], seq in [1, max_seq]");
     IRO_REQUIRE(c->layers[layer].loaded, IRODORI_ERR_NOT_LOADED, "block weights of the layer not loaded");
     IRO_HIP_CHECK(hipSetDevice(c->device));
-    const int D = g.model_dim, L = g.num_layers;
-    IRO_TRY(ensure_nvec(c, B));
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
-    // The caller's vectors in table rows 0..B-1 of (layer, mlp); the table is rebuilt by
-    // the next forward or sampling call.
-    launch_put_mod_vectors(shift, scale, gate, B, D, L, layer, 1, c->tab, st);
+    // All rows in one launch set, each row on its own vectors, read where the caller has them:
+    // the adaLN kernel, W1|W3 with the SwiGLU epilogue, W2 with the gated residual.  (One row at a
+    // time with the norm folded into W1|W3, as a sampler chain runs it, took 110 us for 2 x 750
+    // tokens: nine launches, each for half the rows.)
+    ModTable mt{nullptr, nullptr, 0, 1, g.num_layers};
+    mt.direct[0] = shift;
+    mt.direct[1] = scale;
+    mt.direct[2] = gate;
     PartOpts opt;
     opt.no_next = true;
-    const ModTable one{c->tab, c->zero_step, 0, 1, L};
-    if (c->bf16 && fused_for(c, one, 1)) {
-        // The sampler chain's form, one batch row per launch (each on its own vector): the
-        // operand x (1 + scale) and the row sums, then W1|W3 with the norm folded in and W2
-        // with the gated residual.
-        const int cap = c->nvec_cap, F = c->Fp;
-        bf16* stage = static_cast<bf16*>(c->shift_stage);
-        launch_shift_stage(c->tab, B, cap, L, D, stage, st);
-        GemmArgs<bf16> ga{};
-        ga.A = stage + (size_t)(layer * 2 + 1) * cap * D;
-        ga.W = static_cast<const bf16*>(c->layers[layer].w13);
-        ga.w_tiled = c->w_tiled;
-        ga.M = B;
-        ga.N = 2 * F;
-        ga.K = D;
-        ga.S = B;
-        ga.C = c->bias13 + (size_t)layer * cap * 2 * F;
-        IRO_REQUIRE(launch_gemm<bf16>(EPI_STORE, ga, st) == 0, IRODORI_ERR_SHAPE, "shift bias gemm shape");
-        for (int b = 0; b < B; b++) {
-            ModTable mt{c->tab, c->zero_step, 0, 1, L, 0, b};
-            const size_t tok0 = (size_t)b * S;
-            opt.x = x + tok0 * D;
-            launch_mod_stats<bf16>(opt.x, static_cast<bf16*>(c->h) + tok0 * D, S, S, D, mt, layer, 1,
-                                   c->rstat + tok0 * (D / 32), st);
-            IRO_TRY(enqueue_part<bf16>(c, layer, 1, S, mt, PART_W13, b, st, opt));
-            IRO_TRY(enqueue_part<bf16>(c, layer, 1, S, mt, PART_W2, b, st, opt));
-        }
-    } else {
-        // All rows in one launch set, each row on its own vector (rows_per_vec 1): the adaLN
-        // kernel, W1|W3 with the SwiGLU epilogue, W2 with the gated residual.
-        opt.x = x;
-        for (int part : {PART_NORM_MLP, PART_W13, PART_W2}) {
-            if (c->bf16)
-                IRO_TRY(enqueue_part<bf16>(c, layer, B, S, one, part, 0, st, opt));
-            else
-                IRO_TRY(enqueue_part<float>(c, layer, B, S, one, part, 0, st, opt));
-        }
+    opt.unfused = true;
+    opt.x = x;
+    for (int part : {PART_NORM_MLP, PART_W13, PART_W2}) {
+        if (c->bf16)
+            IRO_TRY(enqueue_part<bf16>(c, layer, B, S, mt, part, 0, st, opt));
+        else
+            IRO_TRY(enqueue_part<float>(c, layer, B, S, mt, part, 0, st, opt));
     }
     return check_launch("swiglu mlp operator");
     IRO_GUARD_END

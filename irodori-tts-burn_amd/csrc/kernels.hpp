@@ -18,10 +18,12 @@ struct ModTable {
     int rows_per_vec;  // batch rows sharing one vector
     int layers;
     int step_add = 0;  // evaluation offset (1: the Heun corrector at t_{i+1})
-    int vec_base = 0;  // first vector (a launch over one batch row of a multi-row table)
+    // Set: the vectors of the launch's one (layer, kind) are [batch rows, D] arrays of the caller
+    // (shift, scale, gate), row b on its own; the table is not read.
+    const float* direct[3] = {nullptr, nullptr, nullptr};
 };
 __host__ __device__ inline int mod_vec_index(const ModTable& mt, int step, int b) {
-    return (step + mt.step_add) * mt.step_stride + b / mt.rows_per_vec + mt.vec_base;
+    return (step + mt.step_add) * mt.step_stride + b / mt.rows_per_vec;
 }
 
 // Position of latent/context key s inside a V^T row.  bf16 path (32x32x16 attention):
@@ -189,11 +191,6 @@ void launch_attn_op_stage(const float* q, const float* k, const float* v, const 
                           float eps, float q_scale, int vt_stride, T* Q, T* K, T* Vt, T* G, hipStream_t st);
 template <typename T>
 void launch_to_f32(const T* src, long n, float* dst, hipStream_t st);
-// Modulation vectors [B, D] (shift, scale, gate as applied) into table rows vec b, (layer,
-// kind) of tab [vec][layer][2][3][D].
-void launch_put_mod_vectors(const float* shift, const float* scale, const float* gate, int B, int D, int layers,
-                            int layer, int kind, float* tab, hipStream_t st);
-
 // ---- kernels_cond.hip ------------------------------------------------------------------
 struct VecLinJob {
     const float* X;  // [nvec, ldx]

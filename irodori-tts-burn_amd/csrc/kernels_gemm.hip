@@ -190,6 +190,7 @@ __device__ __forceinline__ int stage_off_packed(int r, int col) {
 
 __device__ __forceinline__ const float* gate_vec(const ModTable& mt, int b, int layer, int kind,
                                                 int D) {
+    if (mt.direct[2]) return mt.direct[2] + (size_t)b * D;
     int vec = mod_vec_index(mt, mt.step ? *mt.step : 0, b);
     return mt.tab + ((size_t)vec * mt.layers * 6 + (size_t)layer * 6 + kind * 3 + 2) * D;
 }
@@ -358,8 +359,10 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
 #pragma unroll
                 for (int u = 0; u < 2; u++) {
                     const int bb = u ? b_hi : b_lo;
-                    const float* g = a.mt.tab + ((size_t)mod_vec_index(a.mt, step, bb) * a.mt.layers * 6 +
-                                                 (size_t)a.layer * 6 + a.kind * 3 + 2) * a.N;
+                    const float* g = a.mt.direct[2]
+                                         ? a.mt.direct[2] + (size_t)bb * a.N
+                                         : a.mt.tab + ((size_t)mod_vec_index(a.mt, step, bb) * a.mt.layers * 6 +
+                                                       (size_t)a.layer * 6 + a.kind * 3 + 2) * a.N;
 #pragma unroll
                     for (int j = 0; j < FN; j++) gpre[i][u][j] = (!u || need_hi) ? g[n0 + wn0 + 32 * j + cl] : 0.f;
                     if (!F8 && a.Hn) {
@@ -1332,7 +1335,7 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
     if (snake_out && (!a.alpha || a.alpha_n <= 0)) return -1;
     switch (EPI) {
         case EPI_STORE: if (!a.C) return -1; break;
-        case EPI_RESID: if (!a.x || !a.mt.tab) return -1; break;
+        case EPI_RESID: if (!a.x || (!a.mt.tab && !a.mt.direct[2])) return -1; break;
         case EPI_ADD: if (!a.x) return -1; break;
         case EPI_SWIGLU: if (F8 ? (!a.U8 || !a.U8s) : !a.U) return -1; break;
         case EPI_SNAKE: if (!a.U) return -1; break;
@@ -1353,7 +1356,7 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
     if (a.rstat && (F8 || (EPI != EPI_QKVG && EPI != EPI_SWIGLU) || !a.rbias || a.K % 128 || a.K > 2048 ||
                     a.S <= 0 || !a.mt.tab || a.mt.rows_per_vec < (a.M + a.S - 1) / a.S))
         return -1;
-    if (a.Hn && (F8 || EPI != EPI_RESID || !a.rstat_out || a.N % 32 || a.next_layer < 0 ||
+    if (a.Hn && (F8 || EPI != EPI_RESID || !a.mt.tab || !a.rstat_out || a.N % 32 || a.next_layer < 0 ||
                  a.next_layer >= a.mt.layers || a.next_kind < 0 || a.next_kind > 1))
         return -1;
     if ((size_t)BN * a.K * ES > 0xffffffffull || (size_t)BM * a.K * ES > 0xffffffffull) return -1;

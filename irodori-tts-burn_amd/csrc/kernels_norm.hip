@@ -88,9 +88,9 @@ __global__ __launch_bounds__(256) void norm_mod_kernel(const float* __restrict__
     }
     ss = wave_sum(ss);
     float rms = sqrtf(ss / (float)D + eps);
-    const float* base = mod_base(mt, row / S, layer, kind, D);
-    const float* shift = base;
-    const float* scale = base + D;
+    const int b = row / S;
+    const float* shift = mt.direct[0] ? mt.direct[0] + (size_t)b * D : mod_base(mt, b, layer, kind, D);
+    const float* scale = mt.direct[0] ? mt.direct[1] + (size_t)b * D : shift + D;
     // Every chunk's scale / shift loads go out together after the reduction, before the first
     // store (one cache round trip per row, not one per chunk): one straight-line body when D
     // fills the chunks, a guarded one otherwise.

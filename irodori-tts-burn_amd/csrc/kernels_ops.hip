@@ -1,7 +1,5 @@
-// Small kernels of the isolated block operators (irodori_op_joint_attention /
-// irodori_op_swiglu_mlp): staging the caller's attention operands into the layouts the
-// model's QKV+gate epilogue writes, widening the gated attention output to f32, and placing
-// caller modulation vectors in the context's table.
+// Small kernels of the isolated joint attention operator (irodori_op_joint_attention): staging the caller's attention operands into the layouts the
+// model's QKV+gate epilogue writes and widening the gated attention output to f32.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -94,19 +92,6 @@ __global__ __launch_bounds__(256) void to_f32_kernel(const T* __restrict__ src, 
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) dst[i] = to_f32(src[i]);
 }
 
-__global__ __launch_bounds__(256) void put_mod_vectors_kernel(const float* __restrict__ shift,
-                                                              const float* __restrict__ scale,
-                                                              const float* __restrict__ gate, int D, int layers,
-                                                              int layer, int kind, float* __restrict__ tab) {
-    const int b = blockIdx.y;
-    float* row = tab + ((size_t)b * layers * 6 + (size_t)layer * 6 + kind * 3) * D;
-    for (int d = blockIdx.x * 256 + threadIdx.x; d < D; d += gridDim.x * 256) {
-        row[d] = shift[(size_t)b * D + d];
-        row[D + d] = scale[(size_t)b * D + d];
-        row[2 * D + d] = gate[(size_t)b * D + d];
-    }
-}
-
 }  // namespace
 
 template <typename T>
@@ -132,10 +117,5 @@ void launch_to_f32(const T* src, long n, float* dst, hipStream_t st) {
 }
 template void launch_to_f32<bf16>(const bf16*, long, float*, hipStream_t);
 template void launch_to_f32<float>(const float*, long, float*, hipStream_t);
-
-void launch_put_mod_vectors(const float* shift, const float* scale, const float* gate, int B, int D, int layers,
-                            int layer, int kind, float* tab, hipStream_t st) {
-    put_mod_vectors_kernel<<<dim3((D + 255) / 256, B), 256, 0, st>>>(shift, scale, gate, D, layers, layer, kind, tab);
-}
 
 }  // namespace irodori

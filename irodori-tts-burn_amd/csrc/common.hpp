@@ -1,6 +1,7 @@
 // Shared device/host helpers for the gfx950 (CDNA4) kernels of libirodori_hip.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -153,12 +154,52 @@ __device__ __forceinline__ Frag<f16> load_frag<f16>(const f16* p) {
     return f;
 }
 
+// Four floats of a caller's array, which promises the alignment of a float and no more: one
+// 16-byte load or store all the same (gfx950 serves dword-aligned global addresses).
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 load4u(const float* p) {
+    const f32x4_u v = *reinterpret_cast<const f32x4_u*>(p);
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void store4u(float* p, float a, float b, float c, float d) {
+    f32x4_u v;
+    v[0] = a; v[1] = b; v[2] = c; v[3] = d;
+    *reinterpret_cast<f32x4_u*>(p) = v;
+}
+
+// Four values as one store of T.
+template <typename T>
+__device__ __forceinline__ void store4(T* p, float a, float b, float c, float d);
+template <>
+__device__ __forceinline__ void store4<float>(float* p, float a, float b, float c, float d) {
+    *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
+}
+template <>
+__device__ __forceinline__ void store4<bf16>(bf16* p, float a, float b, float c, float d) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    bf16x4 v = {static_cast<bf16>(a), static_cast<bf16>(b), static_cast<bf16>(c),
+                static_cast<bf16>(d)};
+    *reinterpret_cast<bf16x4*>(p) = v;
+}
+
 // ---------------------------------------------------------------------------------
 // Wavefront (64 lanes) reductions.
 // ---------------------------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+// Sum over each row of 16 lanes, by DPP rotations within the row (VALU only).
+__device__ __forceinline__ float row16_sum(float v) {
+    auto rot = [](float x, auto ctrl) {
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    v += rot(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+    v += rot(v, std::integral_constant<int, 0x124>{});  // row_ror:4
+    v += rot(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+    v += rot(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
     return v;
 }
 __device__ __forceinline__ float wave_max(float v) {

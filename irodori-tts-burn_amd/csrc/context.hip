@@ -442,6 +442,7 @@ struct PartOpts {
     float* x = nullptr;
     bool no_next = false;
     bool unfused = false;  // the adaLN kernel whatever mt would allow (an isolated MLP half)
+    float* attn_out = nullptr;  // PART_ATTN at Dh 64: the gated output in f32, [B*S, D]
 };
 
 // One kernel of a DiT block over batch rows [r0, r0 + B) of the context's buffers, on
@@ -567,6 +568,15 @@ int enqueue_part(irodori_ctx* c, int l, int B, int S, const ModTable& mt, int pa
             aa.out_mode = f8 ? 2 : 0;  // fp8: o goes straight to the W_o operand form
             aa.G = gate;
             aa.O = o;
+            if (opt.attn_out) {
+                // (An f32 context's out_mode 0 is that output already.)
+                if constexpr (std::is_same<T, float>::value) {
+                    aa.O = opt.attn_out;
+                } else {
+                    aa.Of = opt.attn_out;
+                    aa.out_mode = 3;
+                }
+            }
             aa.O8 = o8;
             aa.O8s = o8s;
             int arc;
@@ -1832,22 +1842,22 @@ int irodori_op_joint_attention(irodori_ctx* c, int layer, int B, int S, const fl
                         "context KV of row " + std::to_string(r) + " not set");
     IRO_HIP_CHECK(hipSetDevice(c->device));
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
-    const int H = g.num_heads, D = g.model_dim, vt = (S + 63) / 64 * 64;
+    const int H = g.num_heads, vt = (S + 63) / 64 * 64;
     const float q_scale = 1.4426950408889634f / sqrtf((float)g.head_dim);
     auto& lb = c->layers[layer];
     ModTable mt{c->tab, c->zero_step, 0, B, g.num_layers};  // not read by the attention
+    PartOpts opt;
+    opt.attn_out = out;
     if (c->bf16) {
         launch_attn_op_stage<bf16>(q, k, v, gate, lb.q_norm, lb.k_norm, c->rope_cos, c->rope_sin, B, S, H, g.norm_eps,
                                    q_scale, vt, static_cast<bf16*>(c->q), static_cast<bf16*>(c->ks),
                                    static_cast<bf16*>(c->vs), static_cast<bf16*>(c->gate), st);
-        IRO_TRY(enqueue_part<bf16>(c, layer, B, S, mt, PART_ATTN, 0, st));
-        launch_to_f32<bf16>(static_cast<const bf16*>(c->o), (long)B * S * D, out, st);
+        IRO_TRY(enqueue_part<bf16>(c, layer, B, S, mt, PART_ATTN, 0, st, opt));
     } else {
         launch_attn_op_stage<float>(q, k, v, gate, lb.q_norm, lb.k_norm, c->rope_cos, c->rope_sin, B, S, H,
                                     g.norm_eps, q_scale, vt, static_cast<float*>(c->q), static_cast<float*>(c->ks),
                                     static_cast<float*>(c->vs), static_cast<float*>(c->gate), st);
-        IRO_TRY(enqueue_part<float>(c, layer, B, S, mt, PART_ATTN, 0, st));
-        launch_to_f32<float>(static_cast<const float*>(c->o), (long)B * S * D, out, st);
+        IRO_TRY(enqueue_part<float>(c, layer, B, S, mt, PART_ATTN, 0, st, opt));
     }
     return check_launch("joint attention operator");
     IRO_GUARD_END

@@ -189,8 +189,6 @@ template <typename T>
 void launch_attn_op_stage(const float* q, const float* k, const float* v, const float* gate, const float* q_norm,
                           const float* k_norm, const float* rope_cos, const float* rope_sin, int B, int S, int H,
                           float eps, float q_scale, int vt_stride, T* Q, T* K, T* Vt, T* G, hipStream_t st);
-template <typename T>
-void launch_to_f32(const T* src, long n, float* dst, hipStream_t st);
 // ---- kernels_cond.hip ------------------------------------------------------------------
 struct VecLinJob {
     const float* X;  // [nvec, ldx]
@@ -391,7 +389,9 @@ struct AttnArgs {
     // epilogue: out_mode 0 -> O [B*Sq, H*Dh] (T) = gate[m, h*Dh+d] * attn;
     //           out_mode 1 -> Of [B, H, Sq, Dh] f32;
     //           out_mode 2 -> the out_mode 0 values in the fp8 GEMM-operand form: e4m3
-    //           codes O8 [B*Sq, H*Dh] and E8M0 scales O8s [B*Sq, H*Dh/32] (bf16 kernel only)
+    //           codes O8 [B*Sq, H*Dh] and E8M0 scales O8s [B*Sq, H*Dh/32] (bf16 kernel only);
+    //           out_mode 3 -> the out_mode 0 values unrounded, Of [B*Sq, H*Dh] f32, float-aligned
+    //           (launch_attention32, which takes all modes but 1; launch_attention takes 0 and 1)
     int out_mode;
     const T* G;
     T* O;

@@ -170,27 +170,9 @@ __device__ __forceinline__ bool merge_parities(unsigned char* smem, int par, int
 
 // Normalise, gate and store one 32-query block: o[db][e] = O[q][32 db + 8 (e / 4) + 4 fh +
 // e % 4] for this lane's query q (lanes l and l ^ 32 hold the two halves of its dims).
-// Gate values of one lane's output dims (out_mode 0): dims 32 db + 8 g4 + 4 fh .. + 3.
-template <typename T>
-struct GateQuads {
-    typedef T T4 __attribute__((ext_vector_type(4)));
-    T4 v[2][4];
-};
-template <typename T>
-__device__ __forceinline__ void load_gate(const AttnArgs<T>& a, GateQuads<T>& g, int b, int hh, int q, int fh) {
-    typedef typename GateQuads<T>::T4 T4;
-    q = q < a.Sq ? q : a.Sq - 1;
-    const T* gp = a.G + ((size_t)b * a.Sq + q) * (a.H * 64) + hh * 64 + 4 * fh;
-#pragma unroll
-    for (int db = 0; db < 2; db++)
-#pragma unroll
-        for (int g4 = 0; g4 < 4; g4++) g.v[db][g4] = *reinterpret_cast<const T4*>(gp + 32 * db + 8 * g4);
-}
-
-// gpre: the lane's gate values loaded ahead (out_mode 0), or null to load them here.
 template <typename T>
 __device__ __forceinline__ void store_block(const AttnArgs<T>& a, const f32x16 (&o)[2], float l_run, int b, int hh,
-                                            size_t bh, int q, int fh, const GateQuads<T>* gpre = nullptr) {
+                                            int q, int fh) {
     const float l = sum_halves(l_run);
     const float inv = l > 0.f ? 1.f / l : 0.f;
     if (q >= a.Sq) return;
@@ -225,33 +207,33 @@ __device__ __forceinline__ void store_block(const AttnArgs<T>& a, const f32x16 (
             return;
         }
     }
-    // Dims 32 db + 8 g4 + 4 fh .. + 3 of query q.  The output mode is uniform: one
-    // straight-line body per mode, the gate loads all issued before the first store.
+    // Dims 32 db + 8 g4 + 4 fh .. + 3 of query q, the gate loads all issued before the first
+    // store.  The output mode is uniform.
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    const size_t base = m * (a.H * 64) + hh * 64 + 4 * fh;
+    T4 g[2][4];
+#pragma unroll
+    for (int db = 0; db < 2; db++)
+#pragma unroll
+        for (int g4 = 0; g4 < 4; g4++) g[db][g4] = *reinterpret_cast<const T4*>(a.G + base + 32 * db + 8 * g4);
+    auto val = [&](int db, int g4, int c) { return o[db][4 * g4 + c] * inv * static_cast<float>(g[db][g4][c]); };
     if (a.out_mode == 0) {
-        typedef typename GateQuads<T>::T4 T4;
-        const size_t base = m * (a.H * 64) + hh * 64 + 4 * fh;
-        GateQuads<T> gl;
-        if (!gpre) load_gate<T>(a, gl, b, hh, q, fh);
-        const GateQuads<T>& g = gpre ? *gpre : gl;
 #pragma unroll
         for (int db = 0; db < 2; db++)
 #pragma unroll
             for (int g4 = 0; g4 < 4; g4++) {
                 T4 ov;
 #pragma unroll
-                for (int c = 0; c < 4; c++)
-                    ov[c] = static_cast<T>(o[db][4 * g4 + c] * inv * static_cast<float>(g.v[db][g4][c]));
+                for (int c = 0; c < 4; c++) ov[c] = static_cast<T>(val(db, g4, c));
                 *reinterpret_cast<T4*>(a.O + base + 32 * db + 8 * g4) = ov;
             }
     } else {
-        float* op = a.Of + ((bh * a.Sq) + q) * 64 + 4 * fh;
 #pragma unroll
         for (int db = 0; db < 2; db++)
 #pragma unroll
             for (int g4 = 0; g4 < 4; g4++)
-                *reinterpret_cast<float4*>(op + 32 * db + 8 * g4) =
-                    make_float4(o[db][4 * g4] * inv, o[db][4 * g4 + 1] * inv, o[db][4 * g4 + 2] * inv,
-                                o[db][4 * g4 + 3] * inv);
+                store4u(a.Of + base + 32 * db + 8 * g4, val(db, g4, 0), val(db, g4, 1), val(db, g4, 2),
+                        val(db, g4, 3));
     }
 }
 
@@ -518,7 +500,7 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
         __syncthreads();
         if (!merge_parities<QB, KVS, 1>(smem, par, qb, lane, &o, &m_run, &l_run)) return;
     }
-    store_block<T>(a, o, l_run, b, hh, bh, q0 + fr, fh);
+    store_block<T>(a, o, l_run, b, hh, q0 + fr, fh);
 }
 
 template <typename T, int QB, int KVS, int NT>
@@ -537,15 +519,15 @@ int launch_attention32_t(const AttnArgs<T>& a, hipStream_t st) {
     if (a.Sq <= 0 || a.len0 <= 0 || !a.v_transposed || !a.prescaled || (a.mask0 && !a.bits0)) return -1;
     if (a.K1 && !a.bits1) return -1;
     if ((a.vstride0 % KT) || (a.K1 && (a.vstride1 % KT))) return -1;
-    if (!std::is_same<T, bf16>::value && a.out_mode == 2) return -1;
+    if (!a.G || (a.out_mode == 0 ? !a.O : a.out_mode == 2 ? !a.O8 || !a.O8s : a.out_mode != 3 || !a.Of)) return -1;
     const int ntiles = (a.len0 + KT - 1) / KT + (a.K1 ? (a.len1 + KT - 1) / KT : 0);
     if (ntiles > kAttnMaxKeyTiles) return -1;  // four tile-list words per lane (16384 keys)
     // 2 query blocks x 2 key parities (4 waves, 64 KB LDS) at every size.  Against 4 x 2:
     // one CFG row of 750 frames 18.2 vs 21.1 us with context keys, 12.3 vs 14.5 us without;
-    // B = 2 rows 42.0 vs 42.2 us per operator call; BASELINE config 5 (32 rows) 340.5 vs
-    // 344.4 ms per RF run.  Every query block's arithmetic is the same in either shape (its
+    // B = 2 rows 42.0 vs 42.2 us per operator call; a 32-row RF run of 750 frames 340.5 vs
+    // 344.4 ms.  Every query block's arithmetic is the same in either shape (its
     // two parities merged in the same order), so the shape never changes an output bit.
-    // One key parity (4 x 1, 32 KB) ran config 5 faster still (323.8 ms) but slower at
+    // One key parity (4 x 1, 32 KB) ran the 32 rows faster still (323.8 ms) but slower at
     // B = 2 (45.2 us), and a size-dependent choice would make a row's result depend on the
     // batch it is launched with.
     // The tile list of up to 4096 keys fits one word per lane; longer key ranges take four

@@ -21,20 +21,6 @@ __device__ __forceinline__ const float* mod_base(const ModTable& mt, int b, int 
     return mt.tab + ((size_t)mod_vec(mt, b) * mt.layers * 6 + (size_t)layer * 6 + kind * 3) * D;
 }
 
-template <typename T>
-__device__ __forceinline__ void store4(T* p, float a, float b, float c, float d);
-template <>
-__device__ __forceinline__ void store4<float>(float* p, float a, float b, float c, float d) {
-    *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
-}
-template <>
-__device__ __forceinline__ void store4<bf16>(bf16* p, float a, float b, float c, float d) {
-    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-    bf16x4 v = {static_cast<bf16>(a), static_cast<bf16>(b), static_cast<bf16>(c),
-                static_cast<bf16>(d)};
-    *reinterpret_cast<bf16x4*>(p) = v;
-}
-
 // Row RMSNorm with weight (rms_norm.rs:161-175 semantics), generic D.
 __global__ __launch_bounds__(256) void rms_norm_op_kernel(const float* __restrict__ x,
                                                           const float* __restrict__ w, int rows,
@@ -101,8 +87,8 @@ __global__ __launch_bounds__(256) void norm_mod_kernel(const float* __restrict__
         for (int j = 0; j < NCH; j++) {
             const int d = lane * 4 + 256 * j;
             if (FULL || d < D) {
-                sc[j] = *reinterpret_cast<const float4*>(scale + d);
-                sh[j] = *reinterpret_cast<const float4*>(shift + d);
+                sc[j] = load4u(scale + d);
+                sh[j] = load4u(shift + d);
             }
         }
 #pragma unroll

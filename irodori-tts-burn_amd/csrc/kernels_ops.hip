@@ -1,5 +1,5 @@
-// Small kernels of the isolated joint attention operator (irodori_op_joint_attention): staging the caller's attention operands into the layouts the
-// model's QKV+gate epilogue writes and widening the gated attention output to f32.
+// The staging kernel of the isolated joint attention operator (irodori_op_joint_attention): the
+// caller's attention operands into the layouts the model's QKV+gate epilogue writes.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -21,64 +21,71 @@ __device__ __forceinline__ int vt_src(int p) {
     return (p & ~31) | (((pp >> 2) & 1) * 16 + (pp >> 3) * 4 + (pp & 3));
 }
 
-// One block per (b, h, 64 tokens): 8 wavefronts x 8 tokens, lane = head dimension, the
-// inputs of a wavefront's 8 tokens loaded together.  The head RMSNorm (norm.rs:60-74) and the interleaved
-// half RoPE (rope.rs:82-135) as the QKV epilogue applies them.  V goes through LDS so that
-// each V^T row (b, h, d) leaves as one contiguous run per 16 keys; keys past S (up to the
-// 64-key boundary) are written as zeros.
+// One block per (b, h, 32 tokens): 16 lanes per token, four head dimensions each, so that a
+// lane holds whole RoPE pairs and the head norm's sum stays in one 16-lane row; every load of
+// the block's two passes goes out first.  The head RMSNorm (norm.rs:60-74) and the
+// interleaved half RoPE (rope.rs:82-135) as the QKV epilogue applies them.  V goes through
+// LDS so that each V^T row (b, h, d) leaves as one run of 32 keys; keys past S (up to the
+// 64-key boundary) are written as zeros.  HBM-bound in principle (2 x 750 tokens of 16 heads:
+// 24.6 MB read and 12.3 MB written, 7 us at copy rate, half of it from cache when the caller has just
+// written its operands); a lane per dimension with 4-byte loads and 6-step shuffles took 17 us.
 template <typename T>
-__global__ __launch_bounds__(512) void attn_op_stage_kernel(
+__global__ __launch_bounds__(256) void attn_op_stage_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ gate, const float* __restrict__ q_norm, const float* __restrict__ k_norm,
-    const float* __restrict__ rope_cos, const float* __restrict__ rope_sin, int B, int S, int H, float eps,
+    const float* __restrict__ rope_cos, const float* __restrict__ rope_sin, int S, int H, float eps,
     float q_scale, int vt_stride, T* __restrict__ Q, T* __restrict__ K, T* __restrict__ Vt, T* __restrict__ G) {
-    __shared__ float vs[64][65];
-    const int d = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int s0 = blockIdx.x * 64, h = blockIdx.y, b = blockIdx.z;
-    const float qn = q_norm ? q_norm[h * 64 + d] : 1.f, kn = k_norm ? k_norm[h * 64 + d] : 1.f;
-    {
-        constexpr int i0 = 0;
-        float xq[8], xk[8], xv[8], xg[8], rc[8], rs[8];
-        const bool rope = h < H / 2;
+    __shared__ float vs[32][68];
+    const int tid = threadIdx.x, d = 4 * (tid & 15);
+    const int s0 = blockIdx.x * 32, h = blockIdx.y, b = blockIdx.z;
+    const bool rope = h < H / 2;
+    float4 xq[2], xk[2], xv[2], xg[2];
+    float2 rc[2], rs[2];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int s = s0 + wave * 8 + u, sc = s < S ? s : S - 1;
-            const size_t in = (((size_t)b * S + sc) * H + h) * 64 + d;
-            xq[u] = q[in];
-            xk[u] = k[in];
-            xv[u] = v[in];
-            xg[u] = gate ? gate[in] : 0.f;
-            rc[u] = rope ? rope_cos[(size_t)sc * 32 + (d >> 1)] : 1.f;
-            rs[u] = rope ? rope_sin[(size_t)sc * 32 + (d >> 1)] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int sl = wave * 8 + i0 + u, s = s0 + sl;
-            if (s >= S) {  // wave-uniform
-                vs[sl][d] = 0.f;
-                continue;
-            }
-            float yq = xq[u], yk = xk[u];
-            if (q_norm) yq *= rsqrtf(wave_sum(yq * yq) * (1.f / 64.f) + eps) * qn;
-            if (k_norm) yk *= rsqrtf(wave_sum(yk * yk) * (1.f / 64.f) + eps) * kn;
-            if (rope) {
-                const float c = rc[u], sn = rs[u];
-                const float pq = __shfl_xor(yq, 1, 64), pk = __shfl_xor(yk, 1, 64);
-                yq = (d & 1) ? pq * sn + yq * c : yq * c - pq * sn;
-                yk = (d & 1) ? pk * sn + yk * c : yk * c - pk * sn;
-            }
-            const size_t o = (((size_t)b * H + h) * S + s) * 64 + d;
-            Q[o] = from_f32<T>(yq * q_scale);
-            K[o] = from_f32<T>(yk);
-            const float gv = gate ? 1.f / (1.f + expf(-xg[u])) : 1.f;
-            G[((size_t)b * S + s) * H * 64 + h * 64 + d] = from_f32<T>(gv);
-            vs[sl][d] = xv[u];
+    for (int u = 0; u < 2; u++) {
+        const int s = s0 + 16 * u + (tid >> 4), sc = s < S ? s : S - 1;
+        const size_t in = (((size_t)b * S + sc) * H + h) * 64 + d;
+        xq[u] = load4u(q + in);
+        xk[u] = load4u(k + in);
+        xv[u] = load4u(v + in);
+        if (gate) xg[u] = load4u(gate + in);
+        rc[u] = make_float2(1.f, 1.f);
+        rs[u] = make_float2(0.f, 0.f);
+        if (rope) {
+            rc[u] = *reinterpret_cast<const float2*>(rope_cos + (size_t)sc * 32 + d / 2);
+            rs[u] = *reinterpret_cast<const float2*>(rope_sin + (size_t)sc * 32 + d / 2);
         }
     }
+    // The head norm and the rotation of a token's four dimensions.
+    auto head = [&](const float4& x, const float* norm, const float2& c, const float2& sn) {
+        float4 y = x;
+        if (norm) {
+            const float r = rsqrtf(row16_sum(x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w) * (1.f / 64.f) + eps);
+            const float4 w = *reinterpret_cast<const float4*>(norm + h * 64 + d);
+            y = make_float4(x.x * (r * w.x), x.y * (r * w.y), x.z * (r * w.z), x.w * (r * w.w));
+        }
+        if (rope)
+            y = make_float4(y.x * c.x - y.y * sn.x, y.x * sn.x + y.y * c.x, y.z * c.y - y.w * sn.y,
+                            y.z * sn.y + y.w * c.y);
+        return y;
+    };
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int sl = 16 * u + (tid >> 4), s = s0 + sl;
+        const float4 yq = head(xq[u], q_norm, rc[u], rs[u]), yk = head(xk[u], k_norm, rc[u], rs[u]);
+        *reinterpret_cast<float4*>(&vs[sl][d]) = s < S ? xv[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+        if (s >= S) continue;
+        const size_t o = (((size_t)b * H + h) * S + s) * 64 + d;
+        store4<T>(Q + o, yq.x * q_scale, yq.y * q_scale, yq.z * q_scale, yq.w * q_scale);
+        store4<T>(K + o, yk.x, yk.y, yk.z, yk.w);
+        auto sig = [&](float x) { return gate ? 1.f / (1.f + expf(-x)) : 1.f; };
+        store4<T>(G + ((size_t)b * S + s) * H * 64 + h * 64 + d, sig(xg[u].x), sig(xg[u].y), sig(xg[u].z),
+                  sig(xg[u].w));
+    }
     __syncthreads();
-    // V^T row (b, h, dd), positions 8 seg .. 8 seg + 7 of this 64-key block.
-    const int dd = threadIdx.x >> 3, seg = threadIdx.x & 7;
-    T row[8];
+    // V^T row (b, h, dd), positions 8 seg .. 8 seg + 7 of this 32-key group.
+    const int dd = tid >> 2, seg = tid & 3;
+    alignas(16) T row[8];
 #pragma unroll
     for (int j = 0; j < 8; j++) row[j] = from_f32<T>(vs[vt_src<T>(8 * seg + j)][dd]);
     T* dst = Vt + (((size_t)b * H + h) * 64 + dd) * vt_stride + s0 + 8 * seg;
@@ -87,20 +94,16 @@ __global__ __launch_bounds__(512) void attn_op_stage_kernel(
     for (int j = 0; j < 8; j += PER) *reinterpret_cast<uint4*>(dst + j) = *reinterpret_cast<const uint4*>(row + j);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void to_f32_kernel(const T* __restrict__ src, long n, float* __restrict__ dst) {
-    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) dst[i] = to_f32(src[i]);
-}
-
 }  // namespace
 
 template <typename T>
 void launch_attn_op_stage(const float* q, const float* k, const float* v, const float* gate, const float* q_norm,
                           const float* k_norm, const float* rope_cos, const float* rope_sin, int B, int S, int H,
                           float eps, float q_scale, int vt_stride, T* Q, T* K, T* Vt, T* G, hipStream_t st) {
-    // vt_stride is S rounded up to 64: every block's V^T columns lie inside it.
-    const dim3 grid((S + 63) / 64, H, B);
-    attn_op_stage_kernel<T><<<grid, 512, 0, st>>>(q, k, v, gate, q_norm, k_norm, rope_cos, rope_sin, B, S, H, eps,
+    // vt_stride is S rounded up to 64: every block's V^T columns lie inside it, and the blocks
+    // past S clear the rest.
+    const dim3 grid(vt_stride / 32, H, B);
+    attn_op_stage_kernel<T><<<grid, 256, 0, st>>>(q, k, v, gate, q_norm, k_norm, rope_cos, rope_sin, S, H, eps,
                                                   q_scale, vt_stride, Q, K, Vt, G);
 }
 template void launch_attn_op_stage<bf16>(const float*, const float*, const float*, const float*, const float*,
@@ -109,13 +112,5 @@ template void launch_attn_op_stage<bf16>(const float*, const float*, const float
 template void launch_attn_op_stage<float>(const float*, const float*, const float*, const float*, const float*,
                                           const float*, const float*, const float*, int, int, int, float, float, int,
                                           float*, float*, float*, float*, hipStream_t);
-
-template <typename T>
-void launch_to_f32(const T* src, long n, float* dst, hipStream_t st) {
-    long blocks = (n + 255) / 256;
-    to_f32_kernel<T><<<(unsigned)(blocks < 4096 ? blocks : 4096), 256, 0, st>>>(src, n, dst);
-}
-template void launch_to_f32<bf16>(const bf16*, long, float*, hipStream_t);
-template void launch_to_f32<float>(const float*, long, float*, hipStream_t);
 
 }  // namespace irodori

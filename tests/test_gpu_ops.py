@@ -115,3 +115,57 @@ def test_swiglu_mlp_op_config3(oracle64, backend, B):
     err, inc = rel_l2(got, ref), rel_l2(got - x, ref - x)
     print(backend.value, "B=%d swiglu mlp op rel L2 %.2e, increment %.2e" % (B, err, inc))
     assert err < TOL[backend] and inc < 2 * TOL[backend]
+
+
+@pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("S", [1, 31, 33, 64, 97])
+def test_joint_attention_op_ragged(oracle64, backend, S):
+    # Lengths around the staging kernel's 32-token blocks and the 64-key tiles; the operands
+    # at an odd float, the least alignment that the entry point's types promise; no gate, too.
+    cfg = one_layer()
+    w = ih.DitWeights.random(cfg, 7, norm_jitter=0.1)
+    B, H, Dh = 3, cfg.num_heads, cfg.head_dim
+    ctx = ih.make_role_context(cfg, B, 40, 30, ["cond"], seed=8)
+    rng = np.random.default_rng(S)
+    ops = [rng.standard_normal((B, S, H, Dh)).astype(np.float32) for _ in range(3)]
+    ops.append(rng.standard_normal((B, S, H * Dh)).astype(np.float32))
+    n = B * S * H * Dh
+    bufs = [dev(np.concatenate([np.zeros(1, np.float32), a.ravel()])) for a in ops]
+    out = torch.full((n + 2,), 7.0, dtype=torch.float32, device="cuda")
+    ptrs = [b.data_ptr() + 4 for b in bufs]
+    with ih.HipInferenceEngine(cfg, backend, max_rows=B, max_seq=S, max_ctx=ctx.t_ctx) as e:
+        e.load_weights(w)
+        e.set_context_kv(ctx)
+        for gate in (True, False):
+            e.joint_attention(0, B, S, *ptrs[:3], ptrs[3] if gate else 0, out.data_ptr() + 4)
+            torch.cuda.synchronize()
+            g = ops[3] if gate else np.full_like(ops[3], 60.0)
+            ref = joint_attention_ref(oracle64, cfg, w.blocks[0], *ops[:3], g, ctx.k[0], ctx.v[0], ctx.mask)
+            o = out.cpu().numpy()
+            assert o[0] == 7.0 and o[-1] == 7.0
+            assert rel_l2(o[1:-1].reshape(ref.shape), ref) < TOL[backend]
+
+
+@pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("B,S", [(3, 1), (3, 31), (2, 33), (3, 130)])
+def test_swiglu_mlp_op_rows_on_their_own_vectors(oracle64, backend, B, S):
+    # Rows shorter than, and not a multiple of, a GEMM tile's row block, so that one block of
+    # the residual epilogue spans two or three rows' gates; vectors at an odd float.
+    cfg = one_layer(eps=1e-6)
+    w = ih.DitWeights.random(cfg, 3)
+    D = cfg.model_dim
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((B, S, D)).astype(np.float32)
+    vec = [rng.standard_normal((B, D)).astype(np.float32) for _ in range(3)]
+    dx = dev(x)
+    bufs = [dev(np.concatenate([np.zeros(1, np.float32), a.ravel()])) for a in vec]
+    with ih.HipInferenceEngine(cfg, backend, max_rows=B, max_seq=S, max_ctx=1) as e:
+        e.load_weights(w)
+        e.swiglu_mlp(0, B, S, dx.data_ptr(), *[b.data_ptr() + 4 for b in bufs])
+        torch.cuda.synchronize()
+    got = dx.cpu().numpy()
+    shift, scale, gate = vec
+    h = oracle64.fused_adaln(x.reshape(B * S, D), scale, shift, B, S, 1e-6)
+    m = oracle64.swiglu(h, w.blocks[0]["w13"], w.blocks[0]["w2"]).reshape(B, S, D).astype(np.float64)
+    ref = x + gate[:, None, :].astype(np.float64) * m
+    assert rel_l2(got, ref) < TOL[backend] and rel_l2(got - x, ref - x) < 2 * TOL[backend]

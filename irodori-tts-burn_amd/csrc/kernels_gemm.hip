@@ -65,6 +65,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, un
     // Raw (stride 0) buffer; dword3 0x00020000 is the gfx9-family data format for raw access.
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
+constexpr int kMaxWindowCols = 1 << 20;  // a tile's f32 rows (at most 256) stay under 2^30 bytes
 __device__ __forceinline__ void buf_load_lds16(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, void* lds) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
 }
@@ -648,24 +649,46 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
             }
         }
     }
+    // f32 rows of the tile (N <= kMaxWindowCols, 32-bit offsets) as one buffer window that ends with the last row: loads past it give
+    // 0 and stores are dropped, so the plain epilogues run without a branch per row (those cost
+    // the 64x64 tiles about 4 us a launch).
+    [[maybe_unused]] auto row_window = [&](float* p) {
+        const int rows = a.M - m0 < BM ? a.M - m0 : BM;
+        return make_rsrc(p + (size_t)m0 * a.N, (unsigned)rows * (unsigned)a.N * 4u);
+    };
+    [[maybe_unused]] auto row_off = [&](int i, int e, int j) {
+        return (unsigned)((rbase - m0 + 32 * i + 8 * (e >> 2) + (e & 3)) * a.N + n0 + wn0 + 32 * j + cl) * 4u;
+    };
     if constexpr (EPI == EPI_STORE) {
-        float* __restrict__ C = a.C;
-        T* __restrict__ U = a.U;
+        if (!snake_out && a.N <= kMaxWindowCols) {
+            const __amdgpu_buffer_rsrc_t rc = row_window(a.C);
 #pragma unroll
-        for (int i = 0; i < FM; i++)
+            for (int i = 0; i < FM; i++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                int row = rbase + 32 * i + 8 * (e >> 2) + (e & 3);
-                if (row >= a.M) continue;
+                for (int e = 0; e < 16; e++)
 #pragma unroll
-                for (int j = 0; j < FN; j++) {
-                    const long lin = (long)row * a.N + n0 + wn0 + 32 * j + cl;
-                    const float v = acc[i][j][e] + bcol[j];
-                    C[lin] = v;
-                    if (snake_out && lin >= a.u_lo && lin < a.u_hi)
-                        U[lin] = from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j]));
+                    for (int j = 0; j < FN; j++)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[i][j][e] + bcol[j]), rc,
+                                                              row_off(i, e, j), 0, 0);
+        } else {
+            float* __restrict__ C = a.C;
+            T* __restrict__ U = a.U;
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int row = rbase + 32 * i + 8 * (e >> 2) + (e & 3);
+                    if (row >= a.M) continue;
+#pragma unroll
+                    for (int j = 0; j < FN; j++) {
+                        const long lin = (long)row * a.N + n0 + wn0 + 32 * j + cl;
+                        const float v = acc[i][j][e] + bcol[j];
+                        C[lin] = v;
+                        if (snake_out && lin >= a.u_lo && lin < a.u_hi)
+                            U[lin] = from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j]));
+                    }
                 }
-            }
+        }
     } else if constexpr (EPI == EPI_ADD) {
         // The residual elements of each 32-row block are loaded together before any store:
         // interleaved with the stores to the same array, every load would wait out the
@@ -673,16 +696,28 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
         // the registers and the extra loads compete with the operand stream.)
         float* __restrict__ xg = a.x;
         T* __restrict__ U = a.U;
+        const __amdgpu_buffer_rsrc_t rx = row_window(xg);
 #pragma unroll
         for (int i = 0; i < FM; i++) {
             float xv[16][FN], rmv[16];
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const int row = rbase + 32 * i + 8 * (e >> 2) + (e & 3);
-                const bool ok = row < a.M;
-                rmv[e] = ok && a.rmask ? a.rmask[row] : 1.f;
+                rmv[e] = 1.f;
+                if (a.rmask) rmv[e] = a.rmask[row < a.M ? row : a.M - 1];
 #pragma unroll
-                for (int j = 0; j < FN; j++) xv[e][j] = ok ? xg[(long)row * a.N + n0 + wn0 + 32 * j + cl] : 0.f;
+                for (int j = 0; j < FN; j++)
+                    xv[e][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, row_off(i, e, j), 0, 0));
+            }
+            if (!snake_out) {
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+                        __builtin_amdgcn_raw_buffer_store_b32(
+                            __builtin_bit_cast(unsigned, (xv[e][j] + (acc[i][j][e] + bcol[j])) * rmv[e]), rx,
+                            row_off(i, e, j), 0, 0);
+                continue;
             }
 #pragma unroll
             for (int e = 0; e < 16; e++) {
@@ -693,7 +728,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
                     const long lin = (long)row * a.N + n0 + wn0 + 32 * j + cl;
                     const float v = (xv[e][j] + (acc[i][j][e] + bcol[j])) * rmv[e];
                     xg[lin] = v;
-                    if (snake_out) U[lin] = from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j]));
+                    U[lin] = from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j]));
                 }
             }
         }
@@ -1336,7 +1371,7 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
     switch (EPI) {
         case EPI_STORE: if (!a.C) return -1; break;
         case EPI_RESID: if (!a.x || (!a.mt.tab && !a.mt.direct[2])) return -1; break;
-        case EPI_ADD: if (!a.x) return -1; break;
+        case EPI_ADD: if (!a.x || a.N > kMaxWindowCols) return -1; break;
         case EPI_SWIGLU: if (F8 ? (!a.U8 || !a.U8s) : !a.U) return -1; break;
         case EPI_SNAKE: if (!a.U) return -1; break;
         case EPI_RESUNIT: if (!a.W2 || !a.x || (a.U && !a.alpha2)) return -1; break;
@@ -1418,9 +1453,19 @@ void launch_tile_rows(const void* src, int N, int row_bytes, void* dst, hipStrea
 //     128x128 -> the choice below: 24 frames 8.30 -> 7.08, 128 frames 8.14 -> 6.01, 256 frames 7.92 ->
 //     6.49, 384 frames 8.14 -> 7.06, 512 frames 8.29 -> 7.90, 640 frames 8.89 -> 8.60; at 750 and beyond
 //     128x128 is the better one (40 steps 45.5 against 45.8 and 47.0 ms).
+//     W1|W3 launches of more 128x128 tiles than the chip holds at once (512) take 192x128: the same two
+//     workgroups per CU, 1.25x the flops per LDS byte (1500 x 5632 x 1024 28.9 -> 24.2 us; 8 steps
+//     of two chains of 1500 rows 14.6 -> 14.8 ms, 2100 rows 19.6 -> 18.9, 6000 rows 52.8 -> 51.3;
+//     with fewer tiles it loses: 1000 rows 10.1 -> 11.3).
 //   * The D-wide residual projections: 64x64 in four stages, 32x64 while that still leaves most
 //     CUs one workgroup at most (8 steps at 128 frames 7.79 -> 7.44, 384 frames 8.14 -> 7.80, 512 frames 8.29 ->
-//     8.55), 128x128 for batches that give two workgroups per CU.
+//     8.55), 128x128 in two stages for batches that give two workgroups per CU; in between, where
+//     those tiles are at most one per CU and leave under half of them idle, 128x128 over eight wavefronts in four
+//     stages (3000 x 1024 x 2816 29.5 -> 21.7 us; two chains of 2250 rows 21.1 -> 20.2 ms per 8 steps).
+//     The encoder's (one stream) also take 128x64 over eight wavefronts (1024 x 1280 x 3328 26.6 ->
+//     21.9 us; in two chains of 1500 rows, which share the CUs, that tile costs 4 %).
+//   * f32 stores (the encoder's QKV+gate, the shift biases): 64x128 over eight wavefronts where
+//     64x64 needs a second round and it does not (256 x 5120 x 1280 13.2 -> 11.2 us).
 template <typename T>
 static bool wide_enough(const GemmArgs<T>& a) {
     return a.N % 128 == 0 && (long)((a.M + 127) / 128) * (a.N / 128) >= 512;
@@ -1438,29 +1483,39 @@ template <typename T, bool F8>
 static int launch_swiglu(const GemmArgs<T>& a, hipStream_t st) {
     if (tile_count(a.M, a.N, 64, 64) <= 256) return launch_cfg<T, 64, 64, 2, 1, 4, EPI_SWIGLU, F8>(a, st);
     if (tile_count(a.M, a.N, 128, 64) <= 352) return launch_cfg<T, 128, 64, 4, 1, 3, EPI_SWIGLU, F8>(a, st);
+    if constexpr (!F8)
+        if (tile_count(a.M, a.N, 128, 128) > 512) return launch_cfg<T, 192, 128, 2, 2, 2, EPI_SWIGLU>(a, st);
     return launch_cfg<T, 128, 128, 2, 2, 2, EPI_SWIGLU, F8>(a, st);
 }
-template <typename T, bool F8>
-static int launch_resid(const GemmArgs<T>& a, hipStream_t st) {
-    if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_RESID, F8>(a, st);
-    if (tile_count(a.M, a.N, 32, 64) <= 192) return launch_cfg<T, 32, 64, 1, 2, 5, EPI_RESID, F8>(a, st);
-    return launch_cfg<T, 64, 64, 2, 2, 4, EPI_RESID, F8>(a, st);
+// The residual projections (N = the model width): the smallest tile that needs no second round.
+template <typename T, int EPI, bool F8>
+static int launch_narrow(const GemmArgs<T>& a, hipStream_t st) {
+    if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI, F8>(a, st);
+    if (tile_count(a.M, a.N, 32, 64) <= 192) return launch_cfg<T, 32, 64, 1, 2, 5, EPI, F8>(a, st);
+    if (tile_count(a.M, a.N, 64, 64) <= 256) return launch_cfg<T, 64, 64, 2, 2, 4, EPI, F8>(a, st);
+    if (EPI == EPI_ADD && tile_count(a.M, a.N, 128, 64) <= 256)
+        return launch_cfg<T, 128, 64, 4, 2, 4, EPI_ADD, F8>(a, st);
+    if (a.N % 128 == 0 && tile_count(a.M, a.N, 128, 128) > 128 && tile_count(a.M, a.N, 128, 128) <= 256)
+        return launch_cfg<T, 128, 128, 4, 2, 4, EPI, F8>(a, st);
+    return launch_cfg<T, 64, 64, 2, 2, 4, EPI, F8>(a, st);
 }
-
+template <typename T, bool F8>
+static int launch_store(const GemmArgs<T>& a, hipStream_t st) {
+    if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_STORE, F8>(a, st);
+    if (a.N % 128 == 0 && tile_count(a.M, a.N, 64, 64) > 256 && tile_count(a.M, a.N, 64, 128) <= 256)
+        return launch_cfg<T, 64, 128, 2, 4, 4, EPI_STORE, F8>(a, st);
+    return launch_cfg<T, 64, 64, 2, 2, 4, EPI_STORE, F8>(a, st);
+}
 template <typename T>
 int launch_gemm(int epi, const GemmArgs<T>& a, hipStream_t st) {
     if ((epi == EPI_STORE || epi == EPI_ADD) && a.U && (!a.alpha || a.alpha_n <= 0)) return -1;
     switch (epi) {
-        case EPI_STORE:
-            if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_STORE>(a, st);
-            return launch_cfg<T, 64, 64, 2, 2, 4, EPI_STORE>(a, st);
-        case EPI_RESID:
-            return launch_resid<T, false>(a, st);
+        case EPI_STORE: return launch_store<T, false>(a, st);
+        case EPI_RESID: return launch_narrow<T, EPI_RESID, false>(a, st);
         case EPI_ADD:
-            if (wide_enough(a)) return launch_cfg<T, 128, 128, 2, 2, 2, EPI_ADD>(a, st);
             if (a.N % 128 != 0 && a.N % 192 == 0 && (long)((a.M + 127) / 128) * (a.N / 192) >= 512)
                 return launch_cfg<T, 128, 192, 2, 2, 2, EPI_ADD>(a, st);
-            return launch_cfg<T, 64, 64, 2, 2, 4, EPI_ADD>(a, st);
+            return launch_narrow<T, EPI_ADD, false>(a, st);
         case EPI_SWIGLU: return launch_swiglu<T, false>(a, st);
         // QKVG / CTXKV: one head per wave, 2 x 2 waves of 64 columns or 4 x 1 of 128.
         case EPI_QKVG:
@@ -1477,11 +1532,8 @@ int launch_gemm(int epi, const GemmArgs<T>& a, hipStream_t st) {
 int launch_gemm_fp8(int epi, const GemmArgs<bf16>& a, hipStream_t st) {
     if (!a.A8 || !a.As || !a.W8 || !a.ws || a.K % 128 != 0) return -1;
     switch (epi) {
-        case EPI_STORE:
-            if (wide_enough(a)) return launch_cfg<bf16, 128, 128, 2, 2, 2, EPI_STORE, true>(a, st);
-            return launch_cfg<bf16, 64, 64, 2, 2, 4, EPI_STORE, true>(a, st);
-        case EPI_RESID:
-            return launch_resid<bf16, true>(a, st);
+        case EPI_STORE: return launch_store<bf16, true>(a, st);
+        case EPI_RESID: return launch_narrow<bf16, EPI_RESID, true>(a, st);
         case EPI_SWIGLU: return launch_swiglu<bf16, true>(a, st);
         case EPI_QKVG: return launch_qkvg<bf16, true>(a, st);
     }

@@ -372,11 +372,18 @@ int ensure_nvec(irodori_ctx* c, int nvec) {
     return IRODORI_OK;
 }
 
+// Whether a forward over B rows with modulation table mt runs the fused adaLN: the bf16
+// context supports it and every row maps to one modulation vector (a sampler evaluation,
+// or a single-row forward).  Decided from (mt, B) alone, so in_proj and every block part
+// of the same forward agree.
+bool fused_for(const irodori_ctx* c, const ModTable& mt, int B) { return c->fused && mt.rows_per_vec >= B; }
+
 // Modulation table for nvec timesteps already in c->tvec (or, when skip_mlp, for cond
-// vectors already in c->cond): tab[v][l][k][ch][:].  With the fused adaLN also the shift
-// biases of layers [l0, l1) (whose weights must be loaded; all layers by default):
+// vectors already in c->cond): tab[v][l][k][ch][:].  shift (set where the blocks that follow run
+// the fused adaLN, fused_for): also the shift biases of layers [l0, l1) (whose weights must be
+// loaded; all layers by default) -- 24 products that a forward of several rows never reads, 0.19 ms:
 // biasq[l][v] = shift_attn(v, l) W_qkvg, bias13[l][v] = shift_mlp(v, l) W13.
-int enqueue_mod_table(irodori_ctx* c, int nvec, bool skip_mlp, bool shift = true, int l0 = 0, int l1 = -1) {
+int enqueue_mod_table(irodori_ctx* c, int nvec, bool skip_mlp, bool shift, int l0 = 0, int l1 = -1) {
     const auto& g = c->cfg;
     int D = g.model_dim, L = g.num_layers, r = g.adaln_rank;
     if (l1 < 0) l1 = L;
@@ -391,7 +398,7 @@ int enqueue_mod_table(irodori_ctx* c, int nvec, bool skip_mlp, bool shift = true
     }
     launch_vec_linear(c->d_jobs_down, L * 6, nvec, r, c->stream);
     launch_vec_linear(c->d_jobs_up, L * 6, nvec, D, c->stream);
-    if (c->fused) {
+    if (shift) {
         const int cap = c->nvec_cap, F = c->Fp;
         bf16* stage = static_cast<bf16*>(c->shift_stage);
         launch_shift_stage(c->tab, nvec, cap, L, D, stage, c->stream);
@@ -414,12 +421,6 @@ int enqueue_mod_table(irodori_ctx* c, int nvec, bool skip_mlp, bool shift = true
     }
     return check_launch("modulation table");
 }
-
-// Whether a forward over B rows with modulation table mt runs the fused adaLN: the bf16
-// context supports it and every row maps to one modulation vector (a sampler evaluation,
-// or a single-row forward).  Decided from (mt, B) alone, so in_proj and every block part
-// of the same forward agree.
-bool fused_for(const irodori_ctx* c, const ModTable& mt, int B) { return c->fused && mt.rows_per_vec >= B; }
 
 // The kernels of one DiT block (diffusion.rs:62-105), in launch order.  The block's
 // first adaLN (attention modulation) is launched by the previous block's PART_NORM_NEXT
@@ -1499,8 +1500,8 @@ static int forward_impl(irodori_ctx* c, int B, int S, const float* x_t, const fl
     IRO_TRY(upload(c, c->tvec, t, sizeof(float) * B));
     IRO_TRY(upload(c, c->xt, x_t, sizeof(float) * (size_t)B * S * P));
     RoctxRange fwd("dit_forward_with_cond_fused");
-    IRO_TRY(enqueue_mod_table(c, B, false));
     ModTable mt{c->tab, c->zero_step, 0, 1, L};
+    IRO_TRY(enqueue_mod_table(c, B, false, fused_for(c, mt, B)));
     {
         RoctxRange range("in_proj");
         IRO_TRY(enqueue_inproj(c, B, S, c->xt, B, 0, mt, c->stream));
@@ -1537,8 +1538,8 @@ int irodori_block_forward(irodori_ctx* c, int layer, int B, int S, float* x, con
     int D = g.model_dim, L = g.num_layers;
     IRO_TRY(ensure_nvec(c, B));
     IRO_TRY(upload(c, c->cond, cond, sizeof(float) * (size_t)B * 3 * D));
-    IRO_TRY(enqueue_mod_table(c, B, true, layer, layer + 1));
     ModTable mt{c->tab, c->zero_step, 0, 1, L};
+    IRO_TRY(enqueue_mod_table(c, B, true, fused_for(c, mt, B), layer, layer + 1));
     size_t n = (size_t)B * S * D;
     IRO_TRY(upload(c, c->x, x, sizeof(float) * n));
     if (fused_for(c, mt, B)) {
@@ -1678,7 +1679,7 @@ static int sample_device_impl(irodori_ctx* c, const irodori_sampler_params* p, i
     }
     IRO_TRY(upload(c, c->plan, plan.data(), sizeof(RfEval) * plan.size()));
     IRO_TRY(upload(c, c->tvec, ts.data(), sizeof(float) * (N + 1)));
-    IRO_TRY(enqueue_mod_table(c, N + 1, false));
+    IRO_TRY(enqueue_mod_table(c, N + 1, false, c->fused));
 
     // Speaker-KV scaling (euler_sampler.rs:258-264, :294-300): the conditioned rows, or in
     // Independent mode every row of the batched cache, in the first max_layers layers.
@@ -1913,7 +1914,7 @@ int irodori_profile_layer(irodori_ctx* c, int B, int S, int iters, irodori_kerne
     IRO_TRY(ensure_nvec(c, 1));
     IRO_TRY(upload(c, c->tvec, t.data(), sizeof(float)));
     IRO_TRY(upload(c, c->xt, x0.data(), sizeof(float) * x0.size()));
-    IRO_TRY(enqueue_mod_table(c, 1, false));
+    IRO_TRY(enqueue_mod_table(c, 1, false, c->fused));
     ModTable mt{c->tab, c->zero_step, 0, B, L};
     IRO_TRY(enqueue_inproj(c, B, S, c->xt, B, 0, mt, c->stream));
     for (int l = 0; l < L; l++) IRO_TRY(enqueue_layer_any(c, l, B, S, mt));  // fills every operand

@@ -22,8 +22,6 @@ __global__ void timestep_embedding_kernel(const float* __restrict__ t, int nvec,
     out[(size_t)v * t_dim + half + i] = sinf(a);
 }
 
-constexpr int kKTile = 64;  // staged X columns per pass
-
 __device__ __forceinline__ float apply_act(float v, int act) {
     if (act == 1) return silu_f(v);
     if (act == 2) return tanhf(v);
@@ -35,15 +33,15 @@ __device__ __forceinline__ float apply_act(float v, int act) {
 // threads are COLS columns x KG = 256 / COLS k-groups: thread (kg, c) owns column
 // n = COLS blockIdx.x + c and the k values k = kg (mod KG), accumulating all VC vectors of
 // the chunk in registers, so W is streamed once per vector chunk (a wavefront reads 64 / COLS
-// row segments of COLS consecutive columns per k).  K advances in tiles of 64: the X tile
+// row segments of COLS consecutive columns per k).  K advances in tiles of KT: the X tile
 // (activation applied) is staged transposed in LDS (one k = VC vectors, broadcast 16-byte
 // reads), and the W and X values of tile t + 1 are loaded into registers while tile t is
 // computed.  The k-groups are summed through LDS at the end, in k-group order.
-template <int VC, int COLS>
+template <int VC, int COLS, int KT>
 __global__ __launch_bounds__(256) void vec_linear_kernel(const VecLinJob* __restrict__ jobs, int nvec) {
-    constexpr int KG = 256 / COLS, NK = kKTile / KG, NX = VC * kKTile / 256;
-    static_assert(VC % 4 == 0 && KG * COLS == 256 && NX * 256 == VC * kKTile, "tile shapes");
-    __shared__ __attribute__((aligned(16))) float xs[kKTile][VC];
+    constexpr int KG = 256 / COLS, NK = KT / KG, NX = VC * KT / 256;
+    static_assert(VC % 4 == 0 && KG * COLS == 256 && NX * 256 == VC * KT, "tile shapes");
+    __shared__ __attribute__((aligned(16))) float xs[KT][VC];
     __shared__ float red[KG - 1][VC][COLS];
     const VecLinJob jb = jobs[blockIdx.y];
     if (blockIdx.x * COLS >= jb.N) return;  // uniform: this job has fewer columns
@@ -57,7 +55,7 @@ __global__ __launch_bounds__(256) void vec_linear_kernel(const VecLinJob* __rest
     for (int v = 0; v < VC; v++) acc[v] = 0.f;
     float wv[NK], xv[NX];
     auto load_tile = [&](int k0) {
-        const int kt = jb.K - k0 < kKTile ? jb.K - k0 : kKTile;
+        const int kt = jb.K - k0 < KT ? jb.K - k0 : KT;
 #pragma unroll
         for (int i = 0; i < NK; i++) {
             const int k = kg + KG * i;
@@ -70,7 +68,7 @@ __global__ __launch_bounds__(256) void vec_linear_kernel(const VecLinJob* __rest
         }
     };
     load_tile(0);
-    for (int k0 = 0; k0 < jb.K; k0 += kKTile) {
+    for (int k0 = 0; k0 < jb.K; k0 += KT) {
         __syncthreads();  // every thread is past the previous tile's X reads
 #pragma unroll
         for (int i = 0; i < NX; i++) {
@@ -81,9 +79,9 @@ __global__ __launch_bounds__(256) void vec_linear_kernel(const VecLinJob* __rest
 #pragma unroll
         for (int i = 0; i < NK; i++) wc[i] = wv[i];
         __syncthreads();
-        if (k0 + kKTile < jb.K) load_tile(k0 + kKTile);  // in flight during this tile
+        if (k0 + KT < jb.K) load_tile(k0 + KT);  // in flight during this tile
         if (active) {
-            const int kt = jb.K - k0 < kKTile ? jb.K - k0 : kKTile;
+            const int kt = jb.K - k0 < KT ? jb.K - k0 : KT;
 #pragma unroll
             for (int i = 0; i < NK; i++) {
                 const int k = kg + KG * i;
@@ -117,10 +115,10 @@ __global__ __launch_bounds__(256) void vec_linear_kernel(const VecLinJob* __rest
     }
 }
 
-template <int VC, int COLS>
+template <int VC, int COLS, int KT>
 void launch_vec_linear_cfg(const VecLinJob* d_jobs, int njobs, int nvec, int max_n, hipStream_t st) {
     dim3 grid((max_n + COLS - 1) / COLS, njobs, (nvec + VC - 1) / VC);
-    vec_linear_kernel<VC, COLS><<<grid, 256, 0, st>>>(d_jobs, nvec);
+    vec_linear_kernel<VC, COLS, KT><<<grid, 256, 0, st>>>(d_jobs, nvec);
 }
 
 // Shift rows of the modulation table [vec][layer][kind][chunk][D] as bf16 GEMM operands:
@@ -144,12 +142,19 @@ void launch_timestep_embedding(const float* t, int nvec, int t_dim, float* out, 
     timestep_embedding_kernel<<<grid, 256, 0, st>>>(t, nvec, t_dim, out);
 }
 
-// Vector chunks of 16 (an RF run's 41 timesteps are three chunks, run side by side).
-// Columns: 64 per block when the jobs x column blocks fill the chip, else 16 per block with
-// 16 k-groups (the cond MLP's single-job launches).
+// Vector chunks of 16 (an RF run's 41 timesteps are three chunks, run side by side) with K in
+// tiles of 64; up to 4 vectors (a forward's rows) leave registers for tiles of 128 or 256, more
+// weight bytes in flight, which is what bounds the pass over the weights (1024 x 1024 in one job
+// 17.5 -> 9.5 us, 72 jobs of 1024 x 256, 75 MB, 41.6 -> 29.6 us, back from 256 27.6 -> 28.8; tiles of 256
+// in 32 columns took 33 and 32).  Columns: 64 per block when the jobs x column blocks fill the
+// chip, else 16 (the cond MLP's single-job launches).  The columns alone fix the order in which
+// a sum's k values are added, so a vector's result does not depend on how many it is launched with.
 void launch_vec_linear(const VecLinJob* d_jobs, int njobs, int nvec, int max_n, hipStream_t st) {
-    if ((long)((max_n + 63) / 64) * njobs >= 256) launch_vec_linear_cfg<16, 64>(d_jobs, njobs, nvec, max_n, st);
-    else launch_vec_linear_cfg<16, 16>(d_jobs, njobs, nvec, max_n, st);
+    const bool wide = (long)((max_n + 63) / 64) * njobs >= 256, few = nvec <= 4;
+    if (wide && few) launch_vec_linear_cfg<4, 64, 128>(d_jobs, njobs, nvec, max_n, st);
+    else if (wide) launch_vec_linear_cfg<16, 64, 64>(d_jobs, njobs, nvec, max_n, st);
+    else if (few) launch_vec_linear_cfg<4, 16, 256>(d_jobs, njobs, nvec, max_n, st);
+    else launch_vec_linear_cfg<16, 16, 64>(d_jobs, njobs, nvec, max_n, st);
 }
 
 }  // namespace irodori

@@ -90,6 +90,26 @@ def test_forward_per_block(oracle64, name, backend):
 
 
 @pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("layer", [0, 2])
+def test_block_forward_single_row(oracle64, backend, layer):
+    # One row: the bf16 context folds its norm into the projections and needs this layer's shift
+    # biases, computed by no earlier call.
+    cfg = dataclasses.replace(ih.cfg_full_rf(), num_layers=3)
+    w = ih.DitWeights.random(cfg, 3, norm_jitter=0.1)
+    ctx = ih.make_role_context(cfg, 1, 12, 8, ["cond"], seed=4)
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((1, 37, cfg.model_dim)).astype(np.float32)
+    cond = rng.standard_normal((1, 3 * cfg.model_dim)).astype(np.float32)
+    with ih.HipInferenceEngine(cfg, backend, max_rows=1, max_seq=37, max_ctx=ctx.t_ctx) as e:
+        e.load_weights(w)
+        e.set_context_kv(ctx)
+        got = e.block_forward(layer, x, cond)
+    ref = oracle64.block_forward(cfg, w.blocks[layer], x, cond, ctx.k[layer], ctx.v[layer], ctx.mask)
+    assert rel_l2(got, ref) < (1e-5 if backend == F32 else 2e-2)
+
+
+
+@pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
 def test_block_forward_matches_oracle(oracle64, backend):
     cfg = ih.cfg_cpu_plumbing()
     w = ih.DitWeights.random(cfg, 5, norm_jitter=0.05)

@@ -12,9 +12,11 @@
 // no LDS round trip for P.  The A operand of that product is V^T with the keys of each
 // 32-key group permuted so that a lane's 8 keys are one contiguous 16-byte read.  In the
 // model path V is stored that way in HBM (by the QKV epilogue and at context ingest), so
-// K and V^T tiles both move HBM -> registers -> LDS as plain 16-byte rows; the operator
-// entry point (V given as [key][d]) transposes while staging instead.
-// Workgroup = 4 wavefronts x 16*QB queries of one (batch row, head); K/V tiles are double
+// K and V^T tiles both move HBM -> registers -> LDS as plain 16-byte rows.  V given as
+// [key][d] (f32 only) is staged as it is and read an element at a time, which the f32 MFMA
+// takes anyway.
+// Workgroup = 4 query blocks of 16*QB queries of one (batch row, head), each on one wavefront
+// (f32: two, a half of every tile's keys each, merged at the end); K/V tiles are double
 // buffered in LDS with register prefetch; context tiles with no valid key are skipped.
 #include "common.hpp"
 #include "kernels.hpp"
@@ -44,49 +46,39 @@ __device__ __forceinline__ Frag<float> lds_frag8<float>(const float* p) {
     return f;
 }
 
-template <typename T>
-__device__ __forceinline__ T vec_elem(const u32x4& v, int e);
-template <>
-__device__ __forceinline__ bf16 vec_elem<bf16>(const u32x4& v, int e) {
-    unsigned w = v[e >> 1];
-    unsigned short u = (e & 1) ? (unsigned short)(w >> 16) : (unsigned short)(w & 0xffff);
-    return __builtin_bit_cast(bf16, u);
-}
-template <>
-__device__ __forceinline__ float vec_elem<float>(const u32x4& v, int e) {
-    // Copy the element into a scalar first: bit-casting the vector-element lvalue
-    // directly reads element 0.
-    unsigned w = v[e];
-    return __builtin_bit_cast(float, w);
-}
-
-// Position of key k (0..63) of a tile inside the transposed V tile.
-__device__ __forceinline__ int vperm(int k) {
-    int c = k >> 5, kk = k & 31;
-    return c * 32 + ((kk & 15) >> 2) * 8 + (kk >> 4) * 4 + (kk & 3);
-}
-
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-template <typename T, int DH, int QB, bool VT, bool PRESCALED>
-__global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
+// Key halves of a tile dealt to separate wavefronts.  f32: two, so that every SIMD has a second
+// wavefront to run its MFMAs (32 cycles each) while the first one is in its softmax or waits for LDS; with
+// one per SIMD the 41 k MFMA cycles of a 64-query workgroup at 631 keys took 100 k.
+template <typename T>
+constexpr int kKeyHalves = sizeof(T) == 4 ? 2 : 1;
+
+// VT: V^T rows and a pre-scaled Q (the model path); else V row-major and Q unscaled.
+template <typename T, int DH, int QB, bool VT>
+__global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a) {
+    constexpr int KVS = kKeyHalves<T>, NT = 256 * KVS, NKB = 4 / KVS;
+    static_assert(VT || sizeof(T) == 4, "row-major V: f32 (16-bit V rows go to kernels_attn_nv.hip)");
     constexpr int VEC = 16 / sizeof(T);
     constexpr int LDK = DH + 16 / sizeof(T);   // K tile row stride
-    constexpr int LDV = KT + 16 / sizeof(T);   // V^T tile row stride
-    constexpr int LOADS = KT * DH / VEC / 256; // 16-byte chunks per thread per K (or V) tile
+    // V^T tile row stride, or V row stride (then 4 rows are 16 banks apart: the four 16-lane groups
+    // of a fragment read cover all 64)
+    constexpr int LDV = VT ? KT + 16 / sizeof(T) : DH + 4;
+    constexpr int LOADS = KT * DH / VEC / NT;  // 16-byte chunks per thread per K (or V) tile
     constexpr int DC = DH / 32, DB = DH / 16;
     constexpr int WQ = 16 * QB;
     static_assert(LOADS >= 1, "tile");
 
     __shared__ __attribute__((aligned(16))) T Ks[2][KT * LDK];
-    __shared__ __attribute__((aligned(16))) T Vt[2][DH * LDV];
+    __shared__ __attribute__((aligned(16))) T Vt[2][(VT ? DH : KT) * LDV];
     __shared__ float Ms[2][KT];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3), half = __builtin_amdgcn_readfirstlane(tid >> 8);
     const int b = blockIdx.z, h = blockIdx.y;
     const int q0 = blockIdx.x * (4 * WQ) + wave * WQ;
     const int fr = lane & 15, g = lane >> 4;
-    const float sl2 = PRESCALED ? 1.0f : a.scale * kLog2e;
+    const float sl2 = VT ? 1.0f : a.scale * kLog2e;
 
     // Q^T fragments (B operand): query q0 + 16*qb + fr, dims 32*dc + 8*g .. +8.
     Frag<T> qf[QB][DC];
@@ -111,12 +103,12 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
     const T* V1b = a.V1 ? a.V1 + bh * (VT ? (size_t)DH * a.vstride1 : (size_t)a.stride1 * DH) : nullptr;
     const float* M0b = a.mask0 ? a.mask0 + (size_t)b * a.len0 : nullptr;
     const float* M1b = a.mask1 ? a.mask1 + (size_t)b * a.stride1 : nullptr;
-    // K chunk c = tid + 256 i: key c / (DH/VEC), elements (c % (DH/VEC)) * VEC..
+    // K chunk c = tid + NT i: key c / (DH/VEC), elements (c % (DH/VEC)) * VEC..
     const int ckey = tid / (DH / VEC), ccol = (tid % (DH / VEC)) * VEC;
-    constexpr int KEY_STEP = 256 / (DH / VEC);
-    // V^T chunk c = tid + 256 i: dim c / (KT/VEC), keys (c % (KT/VEC)) * VEC..
+    constexpr int KEY_STEP = NT / (DH / VEC);
+    // V^T chunk c = tid + NT i: dim c / (KT/VEC), keys (c % (KT/VEC)) * VEC..
     const int vdim = tid / (KT / VEC), vkey = (tid % (KT / VEC)) * VEC;
-    constexpr int DIM_STEP = 256 / (KT / VEC);
+    constexpr int DIM_STEP = NT / (KT / VEC);
 
     u32x4 rk[LOADS], rv[LOADS];
     float rm = 0.f;
@@ -160,9 +152,7 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
                 *reinterpret_cast<u32x4*>(&Vt[buf][(vdim + DIM_STEP * i) * LDV + vkey]) =  \
                     rv[i];                                                                 \
             } else {                                                                       \
-                int pk = vperm(key);                                                       \
-                _Pragma("unroll") for (int e = 0; e < VEC; e++)                            \
-                    Vt[buf][(ccol + e) * LDV + pk] = vec_elem<T>(rv[i], e);                \
+                *reinterpret_cast<u32x4*>(&Vt[buf][key * LDV + ccol]) = rv[i];             \
             }                                                                              \
         }                                                                                  \
         if (tid < KT) Ms[buf][tid] = rm;                                                   \
@@ -192,15 +182,15 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
         const T* ks = Ks[buf];
         const T* vt = Vt[buf];
 
-        // S^T = K Q^T for the 64 keys of this tile.
-        f32x4 s[4][QB];
+        // S^T = K Q^T for this wavefront's keys of the tile: 64, or the 32 of its half.
+        f32x4 s[NKB][QB];
 #pragma unroll
-        for (int kb = 0; kb < 4; kb++) {
+        for (int kb = 0; kb < NKB; kb++) {
 #pragma unroll
             for (int qb = 0; qb < QB; qb++) s[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int dc = 0; dc < DC; dc++) {
-                Frag<T> kf = lds_frag8<T>(ks + (kb * 16 + fr) * LDK + dc * 32 + g * 8);
+                Frag<T> kf = lds_frag8<T>(ks + ((half * NKB + kb) * 16 + fr) * LDK + dc * 32 + g * 8);
 #pragma unroll
                 for (int qb = 0; qb < QB; qb++) mma16(s[kb][qb], kf, qf[qb][dc]);
             }
@@ -208,21 +198,21 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
         // Online softmax over this tile (log2 domain), per query column.  Latent self
         // tiles are never masked except past the segment end (last tile only).
         const bool masked = t >= nt0 || (t + 1) * KT > a.len0 || M0b != nullptr;
-        float bias[4][4];
+        float bias[NKB][4];
         if (masked) {
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++)
+            for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) bias[kb][i] = Ms[buf][kb * 16 + 4 * g + i];
+                for (int i = 0; i < 4; i++) bias[kb][i] = Ms[buf][(half * NKB + kb) * 16 + 4 * g + i];
         }
 #pragma unroll
         for (int qb = 0; qb < QB; qb++) {
             float mx = -INFINITY;
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++)
+            for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    float v = PRESCALED ? s[kb][qb][i] : s[kb][qb][i] * sl2;
+                    float v = VT ? s[kb][qb][i] : s[kb][qb][i] * sl2;
                     if (masked) v += bias[kb][i];
                     s[kb][qb][i] = v;
                     mx = fmaxf(mx, v);
@@ -234,7 +224,7 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
             float corr = fast_exp2(m_run[qb] - m_use);
             float psum = 0.f;
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++)
+            for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     float p = fast_exp2(s[kb][qb][i] - m_use);
@@ -248,7 +238,8 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
         }
         // O^T += V^T P^T, 32 keys per MFMA.
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
+        for (int c = 0; c < 2 / KVS; c++) {
+            const int kc = 32 * (half + c);  // this group's first key (half is 0 with one half)
             Frag<T> pf[QB];
 #pragma unroll
             for (int qb = 0; qb < QB; qb++)
@@ -259,7 +250,14 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
                 }
 #pragma unroll
             for (int d = 0; d < DB; d++) {
-                Frag<T> vf = lds_frag8<T>(vt + (d * 16 + fr) * LDV + c * 32 + g * 8);
+                Frag<T> vf;
+                if constexpr (VT) {
+                    vf = lds_frag8<T>(vt + (d * 16 + fr) * LDV + kc + g * 8);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        vf.v[e] = vt[(kc + 16 * (e >> 2) + 4 * g + (e & 3)) * LDV + d * 16 + fr];
+                }
 #pragma unroll
                 for (int qb = 0; qb < QB; qb++) mma16(o[d][qb], vf, pf[qb]);
             }
@@ -272,6 +270,37 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
 #undef ATTN_NEXT
 #undef ATTN_GLOAD
 #undef ATTN_LSTORE
+
+    // The second half's (m, l, O) into the first's, through the K tiles (every wavefront is past
+    // the last tile's barrier).
+    if constexpr (KVS == 2) {
+        static_assert(sizeof(Ks) >= sizeof(float) * 4 * 64 * (4 * DB + 2), "merge buffer");
+        float* comb = reinterpret_cast<float*>(&Ks[0][0]) + (size_t)wave * 64 * (4 * DB + 2) + lane;
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++) {
+            if (qb) __syncthreads();
+            if (half) {
+#pragma unroll
+                for (int d = 0; d < DB; d++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) comb[(4 * d + i) * 64] = o[d][qb][i];
+                comb[4 * DB * 64] = m_run[qb];
+                comb[(4 * DB + 1) * 64] = l_run[qb];
+            }
+            __syncthreads();
+            if (!half) {
+                const float m1 = comb[4 * DB * 64], l1 = comb[(4 * DB + 1) * 64];
+                const float mt = fmaxf(m_run[qb], m1), mu = mt == -INFINITY ? 0.f : mt;
+                const float c0 = fast_exp2(m_run[qb] - mu), c1 = fast_exp2(m1 - mu);
+#pragma unroll
+                for (int d = 0; d < DB; d++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) o[d][qb][i] = o[d][qb][i] * c0 + comb[(4 * d + i) * 64] * c1;
+                l_run[qb] = l_run[qb] * c0 + l1 * c1;
+            }
+        }
+        if (half) return;
+    }
 
     // Epilogue: normalise, optional sigmoid-gate multiply, store.
     // o[d][qb][i] = O[q = q0 + 16 qb + fr][dim = 16 d + 4 g + i].
@@ -301,14 +330,14 @@ __global__ __launch_bounds__(256) void attn_kernel(AttnArgs<T> a) {
     }
 }
 
-template <typename T, int DH, bool VT, bool PRE>
+template <typename T, int DH, bool VT>
 int launch_q(const AttnArgs<T>& a, int qb, hipStream_t st) {
     int wq = 16 * qb;
     dim3 grid((a.Sq + 4 * wq - 1) / (4 * wq), a.H, a.B);
     if (qb == 1)
-        attn_kernel<T, DH, 1, VT, PRE><<<grid, 256, 0, st>>>(a);
+        attn_kernel<T, DH, 1, VT><<<grid, 256 * kKeyHalves<T>, 0, st>>>(a);
     else
-        attn_kernel<T, DH, 2, VT, PRE><<<grid, 256, 0, st>>>(a);
+        attn_kernel<T, DH, 2, VT><<<grid, 256 * kKeyHalves<T>, 0, st>>>(a);
     return 0;
 }
 
@@ -322,12 +351,12 @@ int launch_attention(const AttnArgs<T>& a, hipStream_t st) {
     if (a.v_transposed && ((a.vstride0 % KT) || (a.K1 && (a.vstride1 % KT)))) return -1;
     long wgs32 = (long)((a.Sq + 127) / 128) * a.H * a.B;
     int qb = wgs32 >= 512 ? 2 : 1;
-    if (a.v_transposed)
-        return a.prescaled ? launch_q<T, DH, true, true>(a, qb, st) : launch_q<T, DH, true, false>(a, qb, st);
-    return a.prescaled ? launch_q<T, DH, false, true>(a, qb, st) : launch_q<T, DH, false, false>(a, qb, st);
+    if (a.v_transposed != a.prescaled) return -1;
+    if (a.v_transposed) return launch_q<T, DH, true>(a, qb, st);
+    if constexpr (sizeof(T) == 4) return launch_q<T, DH, false>(a, qb, st);
+    return -1;
 }
 
-template int launch_attention<bf16, 64>(const AttnArgs<bf16>&, hipStream_t);
 template int launch_attention<bf16, 128>(const AttnArgs<bf16>&, hipStream_t);
 template int launch_attention<float, 64>(const AttnArgs<float>&, hipStream_t);
 template int launch_attention<float, 128>(const AttnArgs<float>&, hipStream_t);

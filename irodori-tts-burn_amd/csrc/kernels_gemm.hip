@@ -65,7 +65,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, un
     // Raw (stride 0) buffer; dword3 0x00020000 is the gfx9-family data format for raw access.
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
-constexpr int kMaxWindowCols = 1 << 20;  // a tile's f32 rows (at most 256) stay under 2^30 bytes
+constexpr int kMaxWindowCols = 1 << 20;    // a tile's f32 rows (at most 256) stay under 2^30 bytes
+constexpr unsigned kPastWindow = 1u << 29;  // an element past every such window, its offset below 2^32
+// Element el of window r (dropped past the window's end).
+__device__ __forceinline__ void buf_store(float v, __amdgpu_buffer_rsrc_t r, unsigned el) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, el * 4u, 0, 0);
+}
+__device__ __forceinline__ void buf_store(bf16 v, __amdgpu_buffer_rsrc_t r, unsigned el) {
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, el * 2u, 0, 0);
+}
 __device__ __forceinline__ void buf_load_lds16(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, void* lds) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
 }
@@ -649,27 +657,63 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
             }
         }
     }
-    // f32 rows of the tile (N <= kMaxWindowCols, 32-bit offsets) as one buffer window that ends with the last row: loads past it give
-    // 0 and stores are dropped, so the plain epilogues run without a branch per row (those cost
-    // the 64x64 tiles about 4 us a launch).
-    [[maybe_unused]] auto row_window = [&](float* p) {
-        const int rows = a.M - m0 < BM ? a.M - m0 : BM;
-        return make_rsrc(p + (size_t)m0 * a.N, (unsigned)rows * (unsigned)a.N * 4u);
+    // The tile's rows of an output (N <= kMaxWindowCols, 32-bit offsets) as one buffer window that
+    // ends with the last row (or element end): loads past it give 0 and stores are dropped, so
+    // these epilogues run without a branch per row (the branches cost the 64x64 tiles about 4 us
+    // a launch, and hid from the compiler which loads a wait is for).
+    constexpr bool WINDOWED = EPI == EPI_STORE || EPI == EPI_ADD || EPI == EPI_SNAKE || EPI == EPI_RESUNIT;
+    [[maybe_unused]] const unsigned win_elems = (unsigned)(a.M - m0 < BM ? a.M - m0 : BM) * (unsigned)a.N;
+    [[maybe_unused]] auto win = [&](auto* p, unsigned end) {
+        return make_rsrc(p + (size_t)m0 * a.N, end * (unsigned)sizeof(*p));
     };
-    [[maybe_unused]] auto row_off = [&](int i, int e, int j) {
-        return (unsigned)((rbase - m0 + 32 * i + 8 * (e >> 2) + (e & 3)) * a.N + n0 + wn0 + 32 * j + cl) * 4u;
+    [[maybe_unused]] auto win_elem = [&](int i, int e, int j) {
+        return (unsigned)((rbase - m0 + 32 * i + 8 * (e >> 2) + (e & 3)) * a.N + n0 + wn0 + 32 * j + cl);
+    };
+    // The f32 residual x of the ADD and RESUNIT epilogues, XB rows a batch: the loads of a batch go
+    // out before the stores of the one before it, since a wait for loads also waits for every older
+    // store.
+    constexpr int XB = 8, NXB = FM * 16 / XB;
+    [[maybe_unused]] float xv[WINDOWED ? 2 : 1][WINDOWED ? XB : 1][FN];
+    [[maybe_unused]] auto load_x = [&](const __amdgpu_buffer_rsrc_t r, int bt) {
+        if constexpr (WINDOWED)
+#pragma unroll
+            for (int e = 0; e < XB; e++)
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    xv[bt & 1][e][j] = __builtin_bit_cast(
+                        float, __builtin_amdgcn_raw_buffer_load_b32(
+                                   r, win_elem(bt * XB / 16, bt * XB % 16 + e, j) * 4u, 0, 0));
     };
     if constexpr (EPI == EPI_STORE) {
-        if (!snake_out && a.N <= kMaxWindowCols) {
-            const __amdgpu_buffer_rsrc_t rc = row_window(a.C);
+        if (a.N <= kMaxWindowCols) {
+            const __amdgpu_buffer_rsrc_t rc = win(a.C, win_elems);
+            if (!snake_out) {
 #pragma unroll
-            for (int i = 0; i < FM; i++)
+                for (int i = 0; i < FM; i++)
 #pragma unroll
-                for (int e = 0; e < 16; e++)
+                    for (int e = 0; e < 16; e++)
 #pragma unroll
-                    for (int j = 0; j < FN; j++)
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[i][j][e] + bcol[j]), rc,
-                                                              row_off(i, e, j), 0, 0);
+                        for (int j = 0; j < FN; j++)
+                            buf_store(acc[i][j][e] + bcol[j], rc, win_elem(i, e, j));
+            } else {
+                // Elements [u_lo, u_hi) of the Snake output.
+                const long t0 = (long)m0 * a.N, lo = a.u_lo - t0, hi = a.u_hi - t0;
+                const unsigned ulo = lo <= 0 ? 0u : lo < (long)win_elems ? (unsigned)lo : win_elems;
+                const unsigned uhi = hi <= 0 ? 0u : hi < (long)win_elems ? (unsigned)hi : win_elems;
+                const __amdgpu_buffer_rsrc_t ru = win(a.U, uhi);
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+#pragma unroll
+                        for (int j = 0; j < FN; j++) {
+                            const float v = acc[i][j][e] + bcol[j];
+                            const unsigned el = win_elem(i, e, j);
+                            buf_store(v, rc, el);
+                            buf_store(from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j])), ru,
+                                      el < ulo ? kPastWindow : el);
+                        }
+            }
         } else {
             float* __restrict__ C = a.C;
             T* __restrict__ U = a.U;
@@ -690,48 +734,40 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
                 }
         }
     } else if constexpr (EPI == EPI_ADD) {
-        // The residual elements of each 32-row block are loaded together before any store:
-        // interleaved with the stores to the same array, every load would wait out the
-        // memory latency on its own.  (Loading them before the main loop measured slower:
-        // the registers and the extra loads compete with the operand stream.)
-        float* __restrict__ xg = a.x;
-        T* __restrict__ U = a.U;
-        const __amdgpu_buffer_rsrc_t rx = row_window(xg);
+        // (Loading x before the main loop measured slower: the registers and the extra loads
+        // compete with the operand stream.)
+        const __amdgpu_buffer_rsrc_t rx = win(a.x, win_elems);
+        load_x(rx, 0);
+        float rmv[FM][16];
 #pragma unroll
-        for (int i = 0; i < FM; i++) {
-            float xv[16][FN], rmv[16];
+        for (int i = 0; i < FM; i++)
 #pragma unroll
             for (int e = 0; e < 16; e++) {
                 const int row = rbase + 32 * i + 8 * (e >> 2) + (e & 3);
-                rmv[e] = 1.f;
-                if (a.rmask) rmv[e] = a.rmask[row < a.M ? row : a.M - 1];
-#pragma unroll
-                for (int j = 0; j < FN; j++)
-                    xv[e][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, row_off(i, e, j), 0, 0));
+                rmv[i][e] = 1.f;
+                if (a.rmask) rmv[i][e] = a.rmask[row < a.M ? row : a.M - 1];
             }
-            if (!snake_out) {
+        auto body = [&](auto snake_c) {
+            [[maybe_unused]] __amdgpu_buffer_rsrc_t ru;
+            if constexpr (decltype(snake_c)::value) ru = win(a.U, win_elems);
 #pragma unroll
-                for (int e = 0; e < 16; e++)
+            for (int bt = 0; bt < NXB; bt++) {
+                if (bt + 1 < NXB) load_x(rx, bt + 1);
 #pragma unroll
-                    for (int j = 0; j < FN; j++)
-                        __builtin_amdgcn_raw_buffer_store_b32(
-                            __builtin_bit_cast(unsigned, (xv[e][j] + (acc[i][j][e] + bcol[j])) * rmv[e]), rx,
-                            row_off(i, e, j), 0, 0);
-                continue;
+                for (int e = 0; e < XB; e++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++) {
+                        const int i = bt * XB / 16, ei = bt * XB % 16 + e;
+                        const float v = (xv[bt & 1][e][j] + (acc[i][j][ei] + bcol[j])) * rmv[i][ei];
+                        buf_store(v, rx, win_elem(i, ei, j));
+                        if constexpr (decltype(snake_c)::value)
+                            buf_store(from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j])), ru,
+                                      win_elem(i, ei, j));
+                    }
             }
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int row = rbase + 32 * i + 8 * (e >> 2) + (e & 3);
-                if (row >= a.M) continue;
-#pragma unroll
-                for (int j = 0; j < FN; j++) {
-                    const long lin = (long)row * a.N + n0 + wn0 + 32 * j + cl;
-                    const float v = (xv[e][j] + (acc[i][j][e] + bcol[j])) * rmv[e];
-                    xg[lin] = v;
-                    U[lin] = from_f32<T>(snake_eval<T>(v, acol[j], arcol[j], hcol[j]));
-                }
-            }
-        }
+        };
+        if (snake_out) body(std::true_type{});
+        else body(std::false_type{});
     } else if constexpr (EPI == EPI_RESUNIT) {
         // Phase 1: s = Snake(acc + bias) into LDS, slice-major (slice kt2 = columns
         // kt2 * BK .. + BK - 1, BM rows of 128 bytes, chunks swizzled as in the operand
@@ -744,6 +780,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
         unsigned char* tl = smem;
         unsigned char* w2l = smem + NK2 * BM * 128;
         __syncthreads();  // every wave is done with the main loop's stages
+        const __amdgpu_buffer_rsrc_t rx = win(a.x, win_elems);
         const __amdgpu_buffer_rsrc_t rW2 = make_rsrc(a.W2, (unsigned)(BN * K2P * ES));
         unsigned voff2[LPW2];
 #pragma unroll
@@ -778,6 +815,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
         for (int kt2 = 0; kt2 < NK2; kt2++) {
             wait_vmcnt<0>();
             __syncthreads();  // W2 slice kt2 has landed; the s tile is complete
+            if (kt2 == NK2 - 1) load_x(rx, 0);  // behind the last slice's MFMAs
             const unsigned char* at = tl + kt2 * BM * 128;
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) {
@@ -810,50 +848,36 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
                 hc2[j] = a.alpha2[2 * a.N + col];
             }
         }
-        // The residual in batches of XB rows (loads issued together, then the stores).  Tiles
-        // that fit two workgroups per CU take four rows (few registers); the 8-wave 256-row
-        // tile runs one workgroup per CU anyway and takes all sixteen (more loads in flight).
-        constexpr int XB = BM >= 256 ? 16 : 4;
-        float* __restrict__ xg = a.x;
-        T* __restrict__ U = a.U;
+        auto body = [&](auto next_c) {
+            [[maybe_unused]] __amdgpu_buffer_rsrc_t ru;
+            if constexpr (decltype(next_c)::value) ru = win(a.U, win_elems);
 #pragma unroll
-        for (int i = 0; i < FM; i++)
+            for (int bt = 0; bt < NXB; bt++) {
+                if (bt + 1 < NXB) load_x(rx, bt + 1);
 #pragma unroll
-            for (int e4 = 0; e4 < 16; e4 += XB) {
-                float xv[XB][FN];
-#pragma unroll
-                for (int e = 0; e < XB; e++) {
-                    const int row = rbase + 32 * i + 8 * ((e4 + e) >> 2) + ((e4 + e) & 3);
-#pragma unroll
-                    for (int j = 0; j < FN; j++)
-                        xv[e][j] = row < a.M ? xg[(long)row * a.N + n0 + wn0 + 32 * j + cl] : 0.f;
-                }
-#pragma unroll
-                for (int e = 0; e < XB; e++) {
-                    const int row = rbase + 32 * i + 8 * ((e4 + e) >> 2) + ((e4 + e) & 3);
-                    if (row >= a.M) continue;
+                for (int e = 0; e < XB; e++)
 #pragma unroll
                     for (int j = 0; j < FN; j++) {
-                        const long lin = (long)row * a.N + n0 + wn0 + 32 * j + cl;
-                        const float v = xv[e][j] + (acc[i][j][e4 + e] + b2[j]);
-                        xg[lin] = v;
-                        if (next) U[lin] = from_f32<T>(snake_eval<T>(v, a2[j], ar2[j], hc2[j]));
+                        const int i = bt * XB / 16, ei = bt * XB % 16 + e;
+                        const float v = xv[bt & 1][e][j] + (acc[i][j][ei] + b2[j]);
+                        buf_store(v, rx, win_elem(i, ei, j));
+                        if constexpr (decltype(next_c)::value)
+                            buf_store(from_f32<T>(snake_eval<T>(v, a2[j], ar2[j], hc2[j])), ru, win_elem(i, ei, j));
                     }
-                }
             }
+        };
+        if (next) body(std::true_type{});
+        else body(std::false_type{});
     } else if constexpr (EPI == EPI_SNAKE) {
-        T* __restrict__ U = a.U;
+        const __amdgpu_buffer_rsrc_t ru = win(a.U, win_elems);
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int row = rbase + 32 * i + 8 * (e >> 2) + (e & 3);
-                if (row >= a.M) continue;
+            for (int e = 0; e < 16; e++)
 #pragma unroll
                 for (int j = 0; j < FN; j++)
-                    U[(size_t)row * a.N + n0 + wn0 + 32 * j + cl] =
-                        from_f32<T>(snake_eval<T>(acc[i][j][e] + bcol[j], acol[j], arcol[j], hcol[j]));
-            }
+                    buf_store(from_f32<T>(snake_eval<T>(acc[i][j][e] + bcol[j], acol[j], arcol[j], hcol[j])), ru,
+                              win_elem(i, e, j));
     } else if constexpr (EPI == EPI_RESID) {
         // x[row, col] += gate[b(row), col] * C, from the values loaded before the main loop.
         // Fused adaLN producer (Hn set): also Hn = x (1 + scale_next) and the sums of x^2 of
@@ -1373,7 +1397,7 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
         case EPI_RESID: if (!a.x || (!a.mt.tab && !a.mt.direct[2])) return -1; break;
         case EPI_ADD: if (!a.x || a.N > kMaxWindowCols) return -1; break;
         case EPI_SWIGLU: if (F8 ? (!a.U8 || !a.U8s) : !a.U) return -1; break;
-        case EPI_SNAKE: if (!a.U) return -1; break;
+        case EPI_SNAKE: if (!a.U || a.N > kMaxWindowCols) return -1; break;
         case EPI_RESUNIT: if (!a.W2 || !a.x || (a.U && !a.alpha2)) return -1; break;
         case EPI_QKVG:
             if (!a.Q || !a.Kd || !a.Vd || !a.G || !a.q_norm || !a.k_norm || !a.rope_cs || a.H <= 0 ||

@@ -140,7 +140,9 @@ __device__ __forceinline__ TileWord tile_word(const float* mask, int len, int nt
 // a second score tile.  Two ring slots: three (96 KB) measured 14.1 against 13.0 us at 1 x 20
 // heads x 750 x 950 and 35 against 21 us at 2 x 16 x 750 x 1381, where the second workgroup per
 // CU is worth more than the second step of lookahead.
-template <typename T, int DH, int QB, int KVS>
+// UNAL: operands at any element's alignment, tiles through registers an element at a time (the
+// 16-byte buffer-to-LDS loads take dword-aligned addresses).
+template <typename T, int DH, int QB, int KVS, bool UNAL>
 __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_nv_kernel(
     AttnArgs<T> a, int nqb) {
     typedef typename Vec8<T>::type V8;
@@ -186,7 +188,14 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
     {
         const T* qp = a.Q + (bh * a.Sq + (q < a.Sq ? q : a.Sq - 1)) * DH + 8 * fh;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) qf[ks] = *reinterpret_cast<const V8*>(qp + 16 * ks);
+        for (int ks = 0; ks < KS; ks++) {
+            if constexpr (UNAL) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) qf[ks][e] = qp[16 * ks + e];
+            } else {
+                qf[ks] = *reinterpret_cast<const V8*>(qp + 16 * ks);
+            }
+        }
     }
     f32x16 o[DB];
 #pragma unroll
@@ -213,10 +222,18 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
                 int li = j * KVS + gi / NI;
                 li = li < nact ? li : nact - 1;
                 const int t = __builtin_amdgcn_readlane(tw.t, li);
-                const __amdgpu_buffer_rsrc_t r = make_rsrc((is_v ? Vb : Kb) + (size_t)t * KT * DH,
-                                                           (unsigned)(a.len0 - t * KT) * (unsigned)ROWB);
-                buf_load_lds16(r, is_v ? voV[ii] : voK[ii],
-                               (is_v ? vring : kring) + (slot * KVS + gi / NI) * TILE + (gi % NI) * 1024);
+                const T* src = (is_v ? Vb : Kb) + (size_t)t * KT * DH;
+                const unsigned bytes = (unsigned)(a.len0 - t * KT) * (unsigned)ROWB;
+                const unsigned vo = is_v ? voV[ii] : voK[ii];
+                unsigned char* dst = (is_v ? vring : kring) + (slot * KVS + gi / NI) * TILE + (gi % NI) * 1024;
+                if constexpr (UNAL) {
+                    V8 x;  // whole rows are in or out of range
+#pragma unroll
+                    for (int e = 0; e < 8; e++) x[e] = vo < bytes ? src[vo / 2 + e] : static_cast<T>(0.f);
+                    *reinterpret_cast<V8*>(dst + 16 * lane) = x;
+                } else {
+                    buf_load_lds16(make_rsrc(src, bytes), vo, dst);
+                }
             }
         };
         issue(false, 0, 0);
@@ -229,6 +246,7 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
             } else {
                 wait_loads<0>();
             }
+            if constexpr (UNAL) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the tiles' LDS writes
             raw_barrier();
             if (par < nact) score_tile<T, DH>(s, kring + par * TILE, fr, fh, qf);
         }
@@ -403,14 +421,14 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
     }
 }
 
-template <typename T, int DH, int QB, int KVS>
+template <typename T, int DH, int QB, int KVS, bool UNAL = false>
 int launch_cfg(const AttnArgs<T>& a, hipStream_t st) {
     constexpr int lds = 4 * KVS * KT * DH * 2;
     static LdsLimit lim;
-    if (set_lds_limit_once(lim, (const void*)attn_nv_kernel<T, DH, QB, KVS>, lds) != hipSuccess) return -2;
+    if (set_lds_limit_once(lim, (const void*)attn_nv_kernel<T, DH, QB, KVS, UNAL>, lds) != hipSuccess) return -2;
     const long wgs = (long)((a.Sq + 32 * QB - 1) / (32 * QB)) * a.H * a.B;
     if (wgs > 0x7fffffffL) return -1;
-    attn_nv_kernel<T, DH, QB, KVS><<<(unsigned)wgs, 64 * QB * KVS, lds, st>>>(a, (a.Sq + 32 * QB - 1) / (32 * QB));
+    attn_nv_kernel<T, DH, QB, KVS, UNAL><<<(unsigned)wgs, 64 * QB * KVS, lds, st>>>(a, (a.Sq + 32 * QB - 1) / (32 * QB));
     return 0;
 }
 
@@ -426,6 +444,8 @@ template <typename T, int DH>
 int launch_attention_nv(const AttnArgs<T>& a, hipStream_t st) {
     if (a.Sq <= 0 || a.len0 <= 0 || a.K1 || a.v_transposed || a.prescaled) return -1;
     if (a.out_mode == 0 ? (!a.G || !a.O) : !a.Of) return -1;
+    if ((reinterpret_cast<uintptr_t>(a.Q) | reinterpret_cast<uintptr_t>(a.K0) | reinterpret_cast<uintptr_t>(a.V0)) & 15)
+        return launch_cfg<T, DH, 2, 2, true>(a, st);
     if (DH == 128 && (long)((a.Sq + 127) / 128) * a.H * a.B >= 160) return launch_cfg<T, DH, 4, 2>(a, st);
     return launch_cfg<T, DH, 2, 2>(a, st);
 }

@@ -385,6 +385,7 @@ struct AttnArgs {
     bool v_transposed;
     int vstride0, vstride1;
     // prescaled: Q already multiplied by scale * log2(e) (the QKV epilogue does this).
+    // launch_attention takes both or, in f32, neither (V row-major [B, H, stride0, Dh]).
     bool prescaled;
     // epilogue: out_mode 0 -> O [B*Sq, H*Dh] (T) = gate[m, h*Dh+d] * attn;
     //           out_mode 1 -> Of [B, H, Sq, Dh] f32;

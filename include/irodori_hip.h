@@ -182,7 +182,8 @@ int irodori_clear_ctx_kv(irodori_ctx* ctx);
 /* Context projections of one layer, JointAttention wk_text / wv_text and wk_speaker /
  * wv_speaker (or the caption pair) (attention.rs:142-147, :183-207): Burn [d_in, H*Dh],
  * no bias.  aux pointers may be NULL when aux_dim is 0.  Every layer must use the same
- * text_dim / aux_dim. */
+ * text_dim / aux_dim; a build with aux keys needs every layer's aux projection
+ * (IRODORI_ERR_NOT_LOADED otherwise). */
 typedef struct irodori_ctx_proj_weights {
     const float* wk_text; /* [text_dim, H*Dh] */
     const float* wv_text;

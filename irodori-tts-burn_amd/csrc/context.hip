@@ -86,7 +86,7 @@ struct LayerBufs {
     // Context projections (wk/wv_text, wk/wv_speaker|caption, attention.rs:142-147): per
     // segment (0 text, 1 aux) [2 H Dh, kpad] = [Wk ; Wv]^T, input dim zero-padded to 64.
     void* w_ctx[2] = {};
-    bool ctx_proj_loaded = false;
+    bool ctx_proj_loaded[2] = {};  // per segment: w_ctx holds this layer's weights (its slab spans every layer's)
     bool loaded = false;
     std::vector<char> row_set;
 };
@@ -1242,7 +1242,7 @@ int irodori_load_ctx_proj_weights(irodori_ctx* c, int layer, int text_dim, int a
         c->ctx_dim[sgm] = K;
         c->ctx_kpad[sgm] = kpad;
     }
-    lb.ctx_proj_loaded = true;
+    for (int sgm = 0; sgm < 2; sgm++) lb.ctx_proj_loaded[sgm] |= dims[sgm] > 0;
     return IRODORI_OK;
     IRO_GUARD_END
 }
@@ -1268,12 +1268,13 @@ int irodori_build_ctx_kv(irodori_ctx* c, int row, int t_text, const float* text_
     IRO_REQUIRE(t_text == 0 || (text_state && text_mask), IRODORI_ERR_INVALID_ARG, "null text state / mask");
     IRO_REQUIRE(t_aux == 0 || (aux_state && aux_mask), IRODORI_ERR_INVALID_ARG, "null aux state / mask");
     for (int l = 0; l < L; l++) {
-        IRO_REQUIRE(c->layers[l].ctx_proj_loaded, IRODORI_ERR_NOT_LOADED,
+        IRO_REQUIRE(c->layers[l].ctx_proj_loaded[0], IRODORI_ERR_NOT_LOADED,
                     "context projections of layer " + std::to_string(l) + " not loaded");
+        IRO_REQUIRE(t_aux == 0 || c->layers[l].ctx_proj_loaded[1], IRODORI_ERR_NOT_LOADED,
+                    "aux context projections of layer " + std::to_string(l) + " not loaded");
         IRO_REQUIRE(c->layers[l].loaded, IRODORI_ERR_NOT_LOADED,
                     "block weights (k_norm) of layer " + std::to_string(l) + " not loaded");
     }
-    IRO_REQUIRE(t_aux == 0 || c->ctx_dim[1] > 0, IRODORI_ERR_NOT_LOADED, "no aux context projection loaded");
     IRO_HIP_CHECK(hipSetDevice(c->device));
     const int T1 = g.max_ctx > 0 ? g.max_ctx : 1, vs1 = (T1 + 63) / 64 * 64;
 

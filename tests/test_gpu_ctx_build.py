@@ -6,11 +6,14 @@ Bars: the f32 path 1e-5 relative L2 on K and V (one f32 GEMM and a head RMSNorm)
 (states and weights rounded to bf16, K and V stored in bf16); forwards as in
 test_gpu_model.py (1e-4 f32, 1e-2 bf16 per block).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import irodori_hip as ih
 from conftest import rel_l2
+from irodori_hip import _lib as L
 
 pytestmark = pytest.mark.gpu
 
@@ -163,3 +166,41 @@ def test_build_errors_are_reported():
         with pytest.raises(ih.IrodoriError) as ei:  # t_ctx differs from the one already set
             e.build_context_kv(1, text[:5], tm[:5])
         assert ei.value.kind == "Shape"
+
+
+def load_layer(e, proj, layer, aux):
+    """One layer's projections through the C ABI, with or without its aux pair."""
+    ptr = [np.ascontiguousarray(proj.layers[layer][k]).ctypes.data_as(C.POINTER(C.c_float)) if aux or k[3:] == "text"
+           else None for k in ("wk_text", "wv_text", "wk_aux", "wv_aux")]
+    rc = e.lib.irodori_load_ctx_proj_weights(e.ctx, layer, proj.text_dim, proj.aux_dim if aux else 0,
+                                             C.byref(L.CtxProjWeightsC(*ptr)))
+    assert rc == 0
+    e._ctx_dims = (proj.text_dim, proj.aux_dim)
+
+
+@pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("missing", [0, 1])
+def test_a_layer_without_its_aux_projection_is_refused(oracle64, backend, missing):
+    # One layer has only its text pair, the others both (in either order; also what an interrupted
+    # second load leaves): text-only builds run, builds with aux keys are refused until it is loaded.
+    cfg = ih.cfg_tiny()
+    w = ih.DitWeights.random(cfg, 11, std=0.05, norm_jitter=0.1)
+    proj = ih.CtxProjWeights.random(cfg, 40, 72, seed=4, std=0.1)
+    rng = np.random.default_rng(5)
+    text, tm = states(rng, 10, 40, 7)
+    aux, am = states(rng, 9, 72, 9)
+    with ih.HipInferenceEngine(cfg, backend, max_rows=1, max_seq=16, max_ctx=19) as e:
+        e.load_weights(w)
+        load_layer(e, proj, missing, aux=False)
+        for l in range(cfg.num_layers):
+            if l != missing:
+                load_layer(e, proj, l, aux=True)
+        with pytest.raises(ih.IrodoriError) as ei:
+            e.build_context_kv(0, text, tm, aux, am)
+        assert ei.value.kind == "NotLoaded"
+        e.build_context_kv(0, text, tm)
+        check_readback(e, cfg, oracle_ctx(oracle64, cfg, w, proj, [(text, tm, None, None)]), backend)
+        load_layer(e, proj, missing, aux=True)
+        e.clear_context_kv()
+        e.build_context_kv(0, text, tm, aux, am)
+        check_readback(e, cfg, oracle_ctx(oracle64, cfg, w, proj, [(text, tm, aux, am)]), backend)

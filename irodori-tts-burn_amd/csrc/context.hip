@@ -1282,16 +1282,26 @@ int irodori_build_ctx_kv(irodori_ctx* c, int row, int t_text, const float* text_
     // caller's f32 rows and the key mask staged behind them.
     const int lens[2] = {t_text, t_aux};
     const float* states[2] = {text_state, aux_state};
-    const size_t kmax = std::max(c->ctx_kpad[0], c->ctx_kpad[1]), half = (size_t)T1 * kmax;
-    if (!c->ctx_state) {  // t_text + t_aux <= max_ctx rows of the wider padded input
-        c->ctx_state_bytes = half * (c->esz + sizeof(float)) + T1;
-        IRO_TRY(dev_alloc(c, &c->ctx_state, c->ctx_state_bytes));
+    size_t n_op = 0, n_raw = 0;  // elements of the operand (rows of 64-padded width) and of the f32 rows
+    for (int sgm = 0; sgm < 2; sgm++) {
+        n_op += (size_t)lens[sgm] * c->ctx_kpad[sgm];
+        n_raw += (size_t)lens[sgm] * c->ctx_dim[sgm];
     }
-    IRO_REQUIRE(half * (c->esz + sizeof(float)) + T1 <= c->ctx_state_bytes, IRODORI_ERR_SHAPE,
-                "context states exceed the staging buffer");
+    const size_t need = n_op * c->esz + n_raw * sizeof(float) + t_ctx;
+    if (need > c->ctx_state_bytes) {
+        // max_ctx rows of the widest projection loaded so far: every later build fits, unless a wider
+        // projection is loaded first (once at most, the widths being fixed when loaded; the smaller
+        // buffer stays with the context).
+        const size_t wide = (size_t)T1 * std::max(c->ctx_kpad[0], c->ctx_kpad[1]);
+        const size_t bytes = wide * (c->esz + sizeof(float)) + T1;
+        void* wider = nullptr;
+        IRO_TRY(dev_alloc(c, &wider, bytes));
+        c->ctx_state = wider;
+        c->ctx_state_bytes = bytes;
+    }
     char* const operand = static_cast<char*>(c->ctx_state);
-    float* const raw = reinterpret_cast<float*>(operand + half * c->esz);
-    uint8_t* const d_mask = reinterpret_cast<uint8_t*>(raw + half);
+    float* const raw = reinterpret_cast<float*>(operand + n_op * c->esz);
+    uint8_t* const d_mask = reinterpret_cast<uint8_t*>(raw + n_raw);
     size_t off[2] = {0, 0}, roff = 0, total = 0;
     for (int sgm = 0; sgm < 2; sgm++) {
         const int n = lens[sgm], dim = c->ctx_dim[sgm], kpad = c->ctx_kpad[sgm];

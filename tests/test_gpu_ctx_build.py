@@ -204,3 +204,26 @@ def test_a_layer_without_its_aux_projection_is_refused(oracle64, backend, missin
         e.clear_context_kv()
         e.build_context_kv(0, text, tm, aux, am)
         check_readback(e, cfg, oracle_ctx(oracle64, cfg, w, proj, [(text, tm, aux, am)]), backend)
+
+
+@pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
+def test_wider_aux_projection_loaded_after_a_build(oracle64, backend):
+    # The staging of a text-only build is sized for the text; a wider aux projection loaded afterwards
+    # must not refuse later builds, with or without aux keys.
+    cfg = ih.cfg_tiny()
+    w = ih.DitWeights.random(cfg, 11, std=0.05, norm_jitter=0.1)
+    proj = ih.CtxProjWeights.random(cfg, 40, 200, seed=4, std=0.1)
+    rng = np.random.default_rng(5)
+    text, tm = states(rng, 19, 40, 7)
+    aux, am = states(rng, 15, 200, 9)
+    with ih.HipInferenceEngine(cfg, backend, max_rows=1, max_seq=16, max_ctx=19) as e:
+        e.load_weights(w)
+        for l in range(cfg.num_layers):
+            load_layer(e, proj, l, aux=False)
+        e.build_context_kv(0, text, tm)
+        for l in range(cfg.num_layers):
+            load_layer(e, proj, l, aux=True)
+        for row in ((text, tm, None, None), (text[:4], tm[:4], aux, am)):
+            e.clear_context_kv()
+            e.build_context_kv(0, *row)
+            check_readback(e, cfg, oracle_ctx(oracle64, cfg, w, proj, [row]), backend)

@@ -1302,27 +1302,23 @@ int irodori_build_ctx_kv(irodori_ctx* c, int row, int t_text, const float* text_
     char* const operand = static_cast<char*>(c->ctx_state);
     float* const raw = reinterpret_cast<float*>(operand + n_op * c->esz);
     uint8_t* const d_mask = reinterpret_cast<uint8_t*>(raw + n_raw);
-    size_t off[2] = {0, 0}, roff = 0, total = 0;
-    for (int sgm = 0; sgm < 2; sgm++) {
-        const int n = lens[sgm], dim = c->ctx_dim[sgm], kpad = c->ctx_kpad[sgm];
-        off[sgm] = total;
-        if (n == 0) continue;
-        IRO_TRY(upload(c, raw + roff, states[sgm], sizeof(float) * (size_t)n * dim));
-        if (c->bf16)
-            launch_ctx_states<bf16>(raw + roff, n, dim, kpad, reinterpret_cast<bf16*>(operand) + total, c->stream);
-        else
-            launch_ctx_states<float>(raw + roff, n, dim, kpad, reinterpret_cast<float*>(operand) + total, c->stream);
-        roff += (size_t)n * dim;
-        total += (size_t)n * kpad;
-    }
-    if (t_text) IRO_TRY(upload(c, d_mask, text_mask, t_text));
-    if (t_aux) IRO_TRY(upload(c, d_mask + t_text, aux_mask, t_aux));
-
     const int R = g.max_rows, ntl = vs1 / 64;
     const size_t nk = (size_t)H * T1 * Dh, nv = (size_t)H * Dh * vs1;
     auto& l0 = c->layers[0];
-    auto build = [&](auto tag) -> int {
+    auto enqueue = [&](auto tag) -> int {
         typedef decltype(tag) T;
+        size_t off[2] = {0, 0}, roff = 0, total = 0;
+        for (int sgm = 0; sgm < 2; sgm++) {
+            const int n = lens[sgm], dim = c->ctx_dim[sgm], kpad = c->ctx_kpad[sgm];
+            off[sgm] = total;
+            if (n == 0) continue;
+            IRO_TRY(upload(c, raw + roff, states[sgm], sizeof(float) * (size_t)n * dim));
+            launch_ctx_states<T>(raw + roff, n, dim, kpad, reinterpret_cast<T*>(operand) + total, c->stream);
+            roff += (size_t)n * dim;
+            total += (size_t)n * kpad;
+        }
+        if (t_text) IRO_TRY(upload(c, d_mask, text_mask, t_text));
+        if (t_aux) IRO_TRY(upload(c, d_mask + t_text, aux_mask, t_aux));
         T* const ck = static_cast<T*>(l0.ctx_k) + row * nk;
         T* const cv = static_cast<T*>(l0.ctx_v) + row * nv;
         for (int sgm = 0; sgm < 2; sgm++) {
@@ -1346,8 +1342,11 @@ int irodori_build_ctx_kv(irodori_ctx* c, int row, int t_text, const float* text_
                              (size_t)R * ntl, L, H, Dh, t_ctx, T1, vs1, vt_bf16_order(c), c->stream);
         return check_launch("context KV build");
     };
-    IRO_TRY(c->bf16 ? build(bf16()) : build(float()));
-    IRO_HIP_CHECK(hipStreamSynchronize(c->stream));  // the caller's host buffers are free from here on
+    const int rc = c->bf16 ? enqueue(bf16()) : enqueue(float());
+    // The caller's host buffers are free from here on, whether the build was enqueued whole or not.
+    const hipError_t done = hipStreamSynchronize(c->stream);
+    IRO_TRY(rc);
+    IRO_HIP_CHECK(done);
     for (auto& lb : c->layers) lb.row_set[row] = 1;
     if (c->t_ctx != t_ctx) {
         c->graphs.clear();

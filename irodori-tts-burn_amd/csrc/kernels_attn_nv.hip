@@ -223,7 +223,8 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
                 li = li < nact ? li : nact - 1;
                 const int t = __builtin_amdgcn_readlane(tw.t, li);
                 const T* src = (is_v ? Vb : Kb) + (size_t)t * KT * DH;
-                const unsigned bytes = (unsigned)(a.len0 - t * KT) * (unsigned)ROWB;
+                const int rows = a.len0 - t * KT;  // (of every key left, the window's bytes would wrap at 4 GiB)
+                const unsigned bytes = (unsigned)(rows < KT ? rows : KT) * (unsigned)ROWB;
                 const unsigned vo = is_v ? voV[ii] : voK[ii];
                 unsigned char* dst = (is_v ? vring : kring) + (slot * KVS + gi / NI) * TILE + (gi % NI) * 1024;
                 if constexpr (UNAL) {

@@ -83,3 +83,16 @@ def test_operands_at_any_element_alignment(dtype, Sq, Skv, Dh):
         torch.cuda.synchronize()
         got.append(out.cpu().numpy())
     assert np.isfinite(got[0]).all() and np.array_equal(*got)
+
+
+def test_operands_above_four_gib_per_head():
+    # 2^24 + 1 keys of 128 dims: a tile's byte window taken from all remaining keys wraps at 2^32.  One key
+    # holds all the weight: key 5 of the first tile, whose window would end after key 0.
+    Skv, Dh = 2 ** 24 + 1, 128
+    q = torch.zeros((1, 1, 1, Dh), dtype=torch.bfloat16, device="cuda")
+    k, v = (torch.zeros((1, 1, Skv, Dh), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    q[..., 0], k[0, 0, 5, 0], v[0, 0, 5] = 64.0, 64.0, 3.0
+    out = torch.empty((1, 1, 1, Dh), dtype=torch.float32, device="cuda")
+    ops.sdpa(L.DTYPE_BF16, q.data_ptr(), k.data_ptr(), v.data_ptr(), 0, 1, 1, 1, Skv, Dh, 1.0, out.data_ptr())
+    torch.cuda.synchronize()
+    assert (out == 3.0).all()

@@ -6,9 +6,9 @@
 //   S^T = K Q^T      K tile from LDS (A operand), Q^T in registers (B operand): lane l holds
 //                    query l % 32 and keys 8a + 4 (l / 32) + c of every 16-key group.
 //   softmax          in f32: p = exp2(s c - m) with c = scale log2(e), one FMA and one
-//                    exponential an element.  The reference m is lazy: it moves on the
-//                    wavefront's first valid tile and when a lane's sum of p over a tile shows
-//                    a p that may exceed the slack.
+//                    exponential an element.  The reference m is lazy: a query's first tile with
+//                    a score above -inf sets it, and it moves when a lane's sum of p over a tile
+//                    shows a p that may exceed the slack.
 //   O^T += V^T P^T   P^T is the S^T accumulator; the matching V^T operand (4 consecutive keys
 //                    of one dim per lane, twice) comes out of the row-major V tile by
 //                    ds_read_b64_tr_b16, the transposing LDS read, so V needs no transposed
@@ -203,7 +203,8 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
 #pragma unroll
         for (int e = 0; e < 16; e++) o[db][e] = 0.f;
     float m = 0.f, l_run = 0.f;
-    bool first = true;  // wave-uniform: no tile processed yet
+    bool unset = true;  // m is no reference yet: no tile so far, or only scores of -inf
+    bool first = true;  // any lane's unset
 
     for (int w = 0; 64 * w < nt; w++) {  // 4096 keys at a time
         const TileWord tw = tile_word(mb, a.len0, nt, w, lane);
@@ -298,9 +299,14 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
                 return max_halves(mx[0]);
             };
             if (first) {
-                m = tile_max(0.f);
-                m = m == -INFINITY ? 0.f : m;
-                first = false;
+                // (A query whose scores are all -inf so far adds nothing at any m, and must not keep
+                // one: scores far below it would vanish.)
+                const float t = tile_max(0.f);
+                if (unset && t != -INFINITY) {
+                    m = t;
+                    unset = false;
+                }
+                first = __any(unset);
             }
             if constexpr (LOOK) score_tile<T, DH>(sx, kring + (((j + 1) & 1) * KVS + par) * TILE, fr, fh, qf);
             float psum = 0.f;
@@ -358,7 +364,7 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
 
     // Merge the key parities through LDS [parity - 1][QB][16 DB + 2][64 lanes] in parity order.
     if constexpr (KVS > 1) {
-        float m_run = first ? -INFINITY : m;
+        float m_run = unset ? -INFINITY : m;
         float* comb = reinterpret_cast<float*>(smem) + lane;
         constexpr int PER = (16 * DB + 2) * 64;
         __syncthreads();

@@ -85,6 +85,75 @@ def test_operands_at_any_element_alignment(dtype, Sq, Skv, Dh):
     assert np.isfinite(got[0]).all() and np.array_equal(*got)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("Dh", [64, 128])
+def test_scores_of_minus_infinity(oracle64, dtype, Dh):
+    # A query whose first tiles hold only scores of -inf (k = -inf where q > 0) and whose other scores are
+    # far below zero: its reference must come from the first finite score, or every p underflows.
+    # Queries with q[0] = 0 would see 0 * inf, so the last one has q[0] < 0: scores of +inf, a NaN row.
+    code, tdt, tol = TYPES[dtype]
+    B, H, Sq, Skv = 1, 2, 35, 330
+    rng = np.random.default_rng(Dh)
+    q, k, v = (rng.standard_normal((B, H, n, Dh)).astype(np.float32) for n in (Sq, Skv, Skv))
+    q[..., 0], q[..., 1] = 1.0, 16.0
+    q[:, :, -1, 0] = -1.0
+    k[:, :, :192, 0] = -np.inf
+    k[:, :, 192:, 1] = -160.0
+    dq, dk, dv = (torch.from_numpy(a).to("cuda").to(tdt) for a in (q, k, v))
+    out = torch.full((B, H, Sq, Dh), 7.0, dtype=torch.float32, device="cuda")
+    ops.sdpa(code, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), 0, B, H, Sq, Skv, Dh, Dh ** -0.5, out.data_ptr())
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    # The keys at -inf take no part in a finite row: the oracle on the other ones.
+    qq, kk, vv = (a.float().cpu().numpy() for a in (dq, dk, dv))
+    want = oracle64.sdpa(qq, kk[:, :, 192:], vv[:, :, 192:], np.ones((B, Skv - 192), np.float32), Dh ** -0.5)
+    assert np.isfinite(got[:, :, :-1]).all() and np.isnan(got[:, :, -1]).all()
+    assert rel_l2(got[:, :, :-1], want[:, :, :-1]) < tol
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("Dh", [64, 128])
+def test_nan_and_infinite_operands(dtype, Dh):
+    # A masked key's NaN or infinite K row changes nothing; a valid key's makes every row it enters NaN
+    # (an infinite V element only its column).  One query block's NaN row leaves the others alone.
+    code, tdt, _ = TYPES[dtype]
+    B, H, Sq, Skv = 1, 2, 40, 200
+    rng = np.random.default_rng(Dh + 1)
+    q, k, v = (torch.from_numpy(rng.standard_normal((B, H, n, Dh)).astype(np.float32)).to(tdt)
+               for n in (Sq, Skv, Skv))
+    m = torch.ones((B, Skv))
+    m[0, 70:75] = 0
+
+    def run(qq, kk, vv):
+        dq, dk, dv, dm = (a.to("cuda") for a in (qq, kk, vv, m))
+        out = torch.full((B, H, Sq, Dh), 7.0, dtype=torch.float32, device="cuda")
+        ops.sdpa(code, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dm.data_ptr(), B, H, Sq, Skv, Dh, Dh ** -0.5,
+                 out.data_ptr())
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    clean = run(q, k, v)
+    assert np.isfinite(clean).all()
+    bad = k.clone()
+    bad[:, :, 71], bad[:, :, 72], bad[:, :, 73] = float("nan"), float("inf"), float("-inf")
+    assert np.array_equal(run(q, bad, v), clean)
+    for key in (3, 150):
+        bad = k.clone()
+        bad[:, 0, key, 5] = float("nan")
+        got = run(q, bad, v)
+        assert np.isnan(got[:, 0]).all() and np.array_equal(got[:, 1], clean[:, 1])
+    bad = q.clone()
+    bad[:, :, 7] = float("nan")
+    got = run(bad, k, v)
+    rest = np.arange(Sq) != 7
+    assert np.isnan(got[:, :, 7]).all() and np.array_equal(got[:, :, rest], clean[:, :, rest])
+    bad = v.clone()
+    bad[:, :, 9, 11] = float("inf")
+    got = run(q, k, bad)
+    rest = np.arange(Dh) != 11
+    assert (got[..., 11] == np.inf).all() and np.array_equal(got[..., rest], clean[..., rest])
+
+
 def test_operands_above_four_gib_per_head():
     # 2^24 + 1 keys of 128 dims: a tile's byte window taken from all remaining keys wraps at 2^32.  One key
     # holds all the weight: key 5 of the first tile, whose window would end after key 0.

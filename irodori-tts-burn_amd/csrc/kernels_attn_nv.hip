@@ -51,6 +51,8 @@ __device__ __forceinline__ int vswz(int r, int c) {
 }
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
+// 16 bytes at any element's address.
+typedef unsigned u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
 // Four keys k0 .. k0 + 3 of dim d = 32 db + lane % 32, k0 = base + 4 (lane / 32): within each
 // 16-lane group lane i reads 8 bytes of row k0 + i / 4 at dims 16 (group & 1) + 4 (i % 4), and
 // the transposing read hands lane j the group's column j.
@@ -140,8 +142,8 @@ __device__ __forceinline__ TileWord tile_word(const float* mask, int len, int nt
 // a second score tile.  Two ring slots: three (96 KB) measured 14.1 against 13.0 us at 1 x 20
 // heads x 750 x 950 and 35 against 21 us at 2 x 16 x 750 x 1381, where the second workgroup per
 // CU is worth more than the second step of lookahead.
-// UNAL: operands at any element's alignment, tiles through registers an element at a time (the
-// 16-byte buffer-to-LDS loads take dword-aligned addresses).
+// UNAL: operands off a dword boundary, tiles through registers (the 16-byte loads take any
+// address, the buffer-to-LDS ones any dword-aligned address).
 template <typename T, int DH, int QB, int KVS, bool UNAL>
 __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_nv_kernel(
     AttnArgs<T> a, int nqb) {
@@ -188,14 +190,8 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
     {
         const T* qp = a.Q + (bh * a.Sq + (q < a.Sq ? q : a.Sq - 1)) * DH + 8 * fh;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            if constexpr (UNAL) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) qf[ks][e] = qp[16 * ks + e];
-            } else {
-                qf[ks] = *reinterpret_cast<const V8*>(qp + 16 * ks);
-            }
-        }
+        for (int ks = 0; ks < KS; ks++)
+            qf[ks] = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4_u*>(qp + 16 * ks));
     }
     f32x16 o[DB];
 #pragma unroll
@@ -229,10 +225,9 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
                 const unsigned vo = is_v ? voV[ii] : voK[ii];
                 unsigned char* dst = (is_v ? vring : kring) + (slot * KVS + gi / NI) * TILE + (gi % NI) * 1024;
                 if constexpr (UNAL) {
-                    V8 x;  // whole rows are in or out of range
-#pragma unroll
-                    for (int e = 0; e < 8; e++) x[e] = vo < bytes ? src[vo / 2 + e] : static_cast<T>(0.f);
-                    *reinterpret_cast<V8*>(dst + 16 * lane) = x;
+                    u32x4 x = {0, 0, 0, 0};
+                    if (vo < bytes) x = *reinterpret_cast<const u32x4_u*>(src + vo / 2);  // whole rows in or out
+                    *reinterpret_cast<u32x4*>(dst + 16 * lane) = x;
                 } else {
                     buf_load_lds16(make_rsrc(src, bytes), vo, dst);
                 }
@@ -446,12 +441,14 @@ int launch_cfg(const AttnArgs<T>& a, hipStream_t st) {
 // the query blocks per workgroup take four: 31.6 against 46.5 us at 2 x 16 heads x 700 x 1400
 // (192 workgroups), but 13.6 against 11.3 at 1 x 10 x 375 x 375 (30).  64-dim heads lose with
 // four at every size measured (16.6 against 13.2 us at 1 x 20 x 750 x 950).  A query block's
-// arithmetic is the same in either.
+// arithmetic is the same in either.  The line of UNAL is what the buffer-to-LDS loads take: at 1 x
+// 20 x 750 x 950 operands on a dword boundary take 13.1 us (64-dim) and 18.3 (128-dim) as 16-byte
+// aligned ones do, through registers 20.5 and 33.4.
 template <typename T, int DH>
 int launch_attention_nv(const AttnArgs<T>& a, hipStream_t st) {
     if (a.Sq <= 0 || a.len0 <= 0 || a.K1 || a.v_transposed || a.prescaled) return -1;
     if (a.out_mode == 0 ? (!a.G || !a.O) : !a.Of) return -1;
-    if ((reinterpret_cast<uintptr_t>(a.Q) | reinterpret_cast<uintptr_t>(a.K0) | reinterpret_cast<uintptr_t>(a.V0)) & 15)
+    if ((reinterpret_cast<uintptr_t>(a.Q) | reinterpret_cast<uintptr_t>(a.K0) | reinterpret_cast<uintptr_t>(a.V0)) & 3)
         return launch_cfg<T, DH, 2, 2, true>(a, st);
     if (DH == 128 && (long)((a.Sq + 127) / 128) * a.H * a.B >= 160) return launch_cfg<T, DH, 4, 2>(a, st);
     return launch_cfg<T, DH, 2, 2>(a, st);

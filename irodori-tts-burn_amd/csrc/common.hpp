@@ -157,6 +157,7 @@ __device__ __forceinline__ Frag<f16> load_frag<f16>(const f16* p) {
 // Four floats of a caller's array, which promises the alignment of a float and no more: one
 // 16-byte load or store all the same (gfx950 serves dword-aligned global addresses).
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned u32x4_u __attribute__((ext_vector_type(4), aligned(2)));  // and 16 bytes at any 16- or 32-bit element
 __device__ __forceinline__ float4 load4u(const float* p) {
     const f32x4_u v = *reinterpret_cast<const f32x4_u*>(p);
     return make_float4(v[0], v[1], v[2], v[3]);

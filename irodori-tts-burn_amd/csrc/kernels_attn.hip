@@ -88,7 +88,15 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
         int q = q0 + 16 * qb + fr;
         q = q < a.Sq ? q : a.Sq - 1;
 #pragma unroll
-        for (int dc = 0; dc < DC; dc++) qf[qb][dc] = load_frag<T>(qbase + (size_t)q * DH + dc * 32 + g * 8);
+        for (int dc = 0; dc < DC; dc++) {
+            const T* qp = qbase + (size_t)q * DH + dc * 32 + g * 8;
+            if constexpr (VT) {
+                qf[qb][dc] = load_frag<T>(qp);
+            } else {  // a caller's array
+                const float4 lo = load4u(qp), hi = load4u(qp + 4);
+                qf[qb][dc].v = f32x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            }
+        }
     }
 
     const int nt0 = (a.len0 + KT - 1) / KT;
@@ -128,13 +136,13 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
         _Pragma("unroll") for (int i = 0; i < LOADS; i++) {                                \
             int key = key0 + ckey + KEY_STEP * i;                                          \
             key = key < len ? key : len - 1;                                               \
-            rk[i] = *reinterpret_cast<const u32x4*>(kb + (size_t)key * DH + ccol);         \
+            rk[i] = *reinterpret_cast<const u32x4_u*>(kb + (size_t)key * DH + ccol);       \
             if constexpr (VT) {                                                            \
                 const size_t vs = s0 ? a.vstride0 : a.vstride1;                            \
                 rv[i] = *reinterpret_cast<const u32x4*>(                                   \
                     vb + (size_t)(vdim + DIM_STEP * i) * vs + key0 + vkey);                \
             } else {                                                                       \
-                rv[i] = *reinterpret_cast<const u32x4*>(vb + (size_t)key * DH + ccol);     \
+                rv[i] = *reinterpret_cast<const u32x4_u*>(vb + (size_t)key * DH + ccol);   \
             }                                                                              \
         }                                                                                  \
         if (tid < KT) {                                                                    \
@@ -323,8 +331,7 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
                 for (int i = 0; i < 4; i++) op[i] = from_f32<T>(o[d][qb][i] * inv * to_f32(gp[i]));
             } else {
                 float* op = a.Of + (((size_t)b * a.H + h) * a.Sq + q) * DH + dim;
-                *reinterpret_cast<float4*>(op) = make_float4(o[d][qb][0] * inv, o[d][qb][1] * inv,
-                                                             o[d][qb][2] * inv, o[d][qb][3] * inv);
+                store4u(op, o[d][qb][0] * inv, o[d][qb][1] * inv, o[d][qb][2] * inv, o[d][qb][3] * inv);
             }
         }
     }

@@ -51,8 +51,6 @@ __device__ __forceinline__ int vswz(int r, int c) {
 }
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
-// 16 bytes at any element's address.
-typedef unsigned u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
 // Four keys k0 .. k0 + 3 of dim d = 32 db + lane % 32, k0 = base + 4 (lane / 32): within each
 // 16-lane group lane i reads 8 bytes of row k0 + i / 4 at dims 16 (group & 1) + 4 (i % 4), and
 // the transposing read hands lane j the group's column j.
@@ -417,9 +415,8 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
         for (int db = 0; db < DB; db++)
 #pragma unroll
             for (int g4 = 0; g4 < 4; g4++)
-                *reinterpret_cast<float4*>(op + 32 * db + 8 * g4) =
-                    make_float4(o[db][4 * g4] * inv, o[db][4 * g4 + 1] * inv, o[db][4 * g4 + 2] * inv,
-                                o[db][4 * g4 + 3] * inv);
+                store4u(op + 32 * db + 8 * g4, o[db][4 * g4] * inv, o[db][4 * g4 + 1] * inv, o[db][4 * g4 + 2] * inv,
+                        o[db][4 * g4 + 3] * inv);
     }
 }
 

@@ -63,10 +63,10 @@ def test_row_major_attention(oracle64, dtype, B, H, Sq, Skv, Dh, mask, mul):
     assert err < (tol * max(1.0, abs(mul)) if dtype == "f32" else tol)
 
 
-@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
 @pytest.mark.parametrize("Sq,Skv,Dh", [(1, 1, 64), (33, 200, 64), (40, 4161, 64), (65, 193, 128)])
 def test_operands_at_any_element_alignment(dtype, Sq, Skv, Dh):
-    # The same operands one, two or four elements past a 16-byte boundary give the same bits.
+    # The same operands and output one, two or four elements past a 16-byte boundary: the same bits.
     code, tdt, _ = TYPES[dtype]
     B, H = 2, 3
     rng = np.random.default_rng(Skv)
@@ -77,11 +77,13 @@ def test_operands_at_any_element_alignment(dtype, Sq, Skv, Dh):
     got = []
     for off in (0, 1, 2, 4):
         bufs = [torch.from_numpy(np.concatenate([np.zeros(off, np.float32), a])).to("cuda").to(tdt) for a in arrs]
-        out = torch.empty((B, H, Sq, Dh), dtype=torch.float32, device="cuda")
-        ops.sdpa(code, *[b.data_ptr() + 2 * off for b in bufs], dm.data_ptr(), B, H, Sq, Skv, Dh, Dh ** -0.5,
-                 out.data_ptr())
+        out = torch.full((off + B * H * Sq * Dh + 1,), 7.0, dtype=torch.float32, device="cuda")
+        ops.sdpa(code, *[b[off:].data_ptr() for b in bufs], dm.data_ptr(), B, H, Sq, Skv, Dh, Dh ** -0.5,
+                 out[off:].data_ptr())
         torch.cuda.synchronize()
-        got.append(out.cpu().numpy())
+        out = out.cpu().numpy()
+        assert (out[:off] == 7.0).all() and out[-1] == 7.0
+        got.append(out[off:-1])
     assert np.isfinite(got[0]).all()
     for g in got[1:]:
         assert np.array_equal(g, got[0])

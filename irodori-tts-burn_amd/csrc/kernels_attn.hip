@@ -16,7 +16,7 @@
 // [key][d] (f32 only) is staged as it is and read an element at a time, which the f32 MFMA
 // takes anyway.
 // Workgroup = 4 query blocks of 16*QB queries of one (batch row, head), each on one wavefront
-// (f32: two, a half of every tile's keys each, merged at the end); K/V tiles are double
+// (f32: mostly two, a half of every tile's keys each, merged at the end); K/V tiles are double
 // buffered in LDS with register prefetch; context tiles with no valid key are skipped.
 #include "common.hpp"
 #include "kernels.hpp"
@@ -48,16 +48,25 @@ __device__ __forceinline__ Frag<float> lds_frag8<float>(const float* p) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Key halves of a tile dealt to separate wavefronts.  f32: two, so that every SIMD has a second
-// wavefront to run its MFMAs (32 cycles each) while the first one is in its softmax or waits for LDS; with
-// one per SIMD the 41 k MFMA cycles of a 64-query workgroup at 631 keys took 100 k.
+// f32: the two halves of a tile's keys keep their own softmax state (kKeyHalves), merged at the end.
+// They go to separate wavefronts (kKeyWaves), so that every SIMD has a second one to run its MFMAs
+// (32 cycles each) while the first is in its softmax or waits for LDS; with one per SIMD the 41 k
+// MFMA cycles of a 64-query workgroup at 631 keys took 100 k.  Two query blocks of 64 dims on
+// row-major V (launches that fill the chip) leave one wavefront enough to interleave, which then takes both
+// halves, in the same arithmetic and without the merge through LDS: 16 x 16 heads x 750 x 1381 658 -> 602 us, 4 x
+// 32 x 500 x 70 33.2 -> 28.0.  On V^T with its second segment that order is mixed (joint operator, 16 x
+// 512 tokens 268 -> 249 us, but 6 x 700 217 -> 253, 8 x 750 255 -> 286), and for 128 dims it lacks the registers.
 template <typename T>
 constexpr int kKeyHalves = sizeof(T) == 4 ? 2 : 1;
+template <typename T, int DH, int QB, bool VT>
+constexpr int kKeyWaves = DH == 64 && QB == 2 && !VT ? 1 : kKeyHalves<T>;
 
 // VT: V^T rows and a pre-scaled Q (the model path); else V row-major and Q unscaled.
 template <typename T, int DH, int QB, bool VT>
-__global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a) {
-    constexpr int KVS = kKeyHalves<T>, NT = 256 * KVS, NKB = 4 / KVS;
+__global__ __launch_bounds__((256 * kKeyWaves<T, DH, QB, VT>))
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1))) void attn_kernel(AttnArgs<T> a) {
+    constexpr int KH = kKeyHalves<T>, KVS = kKeyWaves<T, DH, QB, VT>, NT = 256 * KVS, NKB = 4 / KH;
+    constexpr int HPW = KH / KVS;  // halves per wavefront
     static_assert(VT || sizeof(T) == 4, "row-major V: f32 (16-bit V rows go to kernels_attn_nv.hip)");
     constexpr int VEC = 16 / sizeof(T);
     constexpr int LDK = DH + 16 / sizeof(T);   // K tile row stride
@@ -166,14 +175,17 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
         if (tid < KT) Ms[buf][tid] = rm;                                                   \
     } while (0)
 
-    f32x4 o[DB][QB];
+    f32x4 oh[HPW][DB][QB];
+    float mh[HPW][QB], lh[HPW][QB];
 #pragma unroll
-    for (int d = 0; d < DB; d++)
+    for (int hp = 0; hp < HPW; hp++)
 #pragma unroll
-        for (int qb = 0; qb < QB; qb++) o[d][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_run[QB], l_run[QB];
+        for (int qb = 0; qb < QB; qb++) {
+            mh[hp][qb] = -INFINITY;
+            lh[hp][qb] = 0.f;
 #pragma unroll
-    for (int qb = 0; qb < QB; qb++) { m_run[qb] = -INFINITY; l_run[qb] = 0.f; }
+            for (int d = 0; d < DB; d++) oh[hp][d][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 
     int t = 0;
     ATTN_NEXT(t);
@@ -190,84 +202,91 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
         const T* ks = Ks[buf];
         const T* vt = Vt[buf];
 
-        // S^T = K Q^T for this wavefront's keys of the tile: 64, or the 32 of its half.
-        f32x4 s[NKB][QB];
 #pragma unroll
-        for (int kb = 0; kb < NKB; kb++) {
+        for (int hp = 0; hp < HPW; hp++) {
+            const int kh = half + hp;
+            auto& o = oh[hp];
+            auto& m_run = mh[hp];
+            auto& l_run = lh[hp];
+            // S^T = K Q^T for the tile's keys: 64, or the 32 of half `kh`.
+            f32x4 s[NKB][QB];
 #pragma unroll
-            for (int qb = 0; qb < QB; qb++) s[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int kb = 0; kb < NKB; kb++) {
 #pragma unroll
-            for (int dc = 0; dc < DC; dc++) {
-                Frag<T> kf = lds_frag8<T>(ks + ((half * NKB + kb) * 16 + fr) * LDK + dc * 32 + g * 8);
+                for (int qb = 0; qb < QB; qb++) s[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int qb = 0; qb < QB; qb++) mma16(s[kb][qb], kf, qf[qb][dc]);
+                for (int dc = 0; dc < DC; dc++) {
+                    Frag<T> kf = lds_frag8<T>(ks + ((kh * NKB + kb) * 16 + fr) * LDK + dc * 32 + g * 8);
+#pragma unroll
+                    for (int qb = 0; qb < QB; qb++) mma16(s[kb][qb], kf, qf[qb][dc]);
+                }
             }
-        }
-        // Online softmax over this tile (log2 domain), per query column.  Latent self
-        // tiles are never masked except past the segment end (last tile only).
-        const bool masked = t >= nt0 || (t + 1) * KT > a.len0 || M0b != nullptr;
-        float bias[NKB][4];
-        if (masked) {
+            // Online softmax over this tile (log2 domain), per query column.  Latent self
+            // tiles are never masked except past the segment end (last tile only).
+            const bool masked = t >= nt0 || (t + 1) * KT > a.len0 || M0b != nullptr;
+            float bias[NKB][4];
+            if (masked) {
 #pragma unroll
-            for (int kb = 0; kb < NKB; kb++)
+                for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) bias[kb][i] = Ms[buf][(half * NKB + kb) * 16 + 4 * g + i];
-        }
+                    for (int i = 0; i < 4; i++) bias[kb][i] = Ms[buf][(kh * NKB + kb) * 16 + 4 * g + i];
+            }
 #pragma unroll
-        for (int qb = 0; qb < QB; qb++) {
-            float mx = -INFINITY;
+            for (int qb = 0; qb < QB; qb++) {
+                float mx = -INFINITY;
 #pragma unroll
-            for (int kb = 0; kb < NKB; kb++)
+                for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    float v = VT ? s[kb][qb][i] : s[kb][qb][i] * sl2;
-                    if (masked) v += bias[kb][i];
-                    s[kb][qb][i] = v;
-                    mx = fmaxf(mx, v);
+                    for (int i = 0; i < 4; i++) {
+                        float v = VT ? s[kb][qb][i] : s[kb][qb][i] * sl2;
+                        if (masked) v += bias[kb][i];
+                        s[kb][qb][i] = v;
+                        mx = fmaxf(mx, v);
+                    }
+                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                float m_new = fmaxf(m_run[qb], mx);
+                float m_use = m_new == -INFINITY ? 0.f : m_new;
+                float corr = fast_exp2(m_run[qb] - m_use);
+                float psum = 0.f;
+#pragma unroll
+                for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        float p = fast_exp2(s[kb][qb][i] - m_use);
+                        s[kb][qb][i] = p;
+                        psum += p;
+                    }
+                l_run[qb] = l_run[qb] * corr + psum;
+                m_run[qb] = m_new;
+#pragma unroll
+                for (int d = 0; d < DB; d++) o[d][qb] *= corr;
+            }
+            // O^T += V^T P^T, 32 keys per MFMA.
+#pragma unroll
+            for (int c = 0; c < 2 / KH; c++) {
+                const int kc = 32 * (kh + c);  // this group's first key (kh is 0 with one half)
+                Frag<T> pf[QB];
+#pragma unroll
+                for (int qb = 0; qb < QB; qb++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        pf[qb].v[i] = from_f32<T>(s[2 * c][qb][i]);
+                        pf[qb].v[4 + i] = from_f32<T>(s[2 * c + 1][qb][i]);
+                    }
+#pragma unroll
+                for (int d = 0; d < DB; d++) {
+                    Frag<T> vf;
+                    if constexpr (VT) {
+                        vf = lds_frag8<T>(vt + (d * 16 + fr) * LDV + kc + g * 8);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            vf.v[e] = vt[(kc + 16 * (e >> 2) + 4 * g + (e & 3)) * LDV + d * 16 + fr];
+                    }
+#pragma unroll
+                    for (int qb = 0; qb < QB; qb++) mma16(o[d][qb], vf, pf[qb]);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            float m_new = fmaxf(m_run[qb], mx);
-            float m_use = m_new == -INFINITY ? 0.f : m_new;
-            float corr = fast_exp2(m_run[qb] - m_use);
-            float psum = 0.f;
-#pragma unroll
-            for (int kb = 0; kb < NKB; kb++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    float p = fast_exp2(s[kb][qb][i] - m_use);
-                    s[kb][qb][i] = p;
-                    psum += p;
-                }
-            l_run[qb] = l_run[qb] * corr + psum;
-            m_run[qb] = m_new;
-#pragma unroll
-            for (int d = 0; d < DB; d++) o[d][qb] *= corr;
-        }
-        // O^T += V^T P^T, 32 keys per MFMA.
-#pragma unroll
-        for (int c = 0; c < 2 / KVS; c++) {
-            const int kc = 32 * (half + c);  // this group's first key (half is 0 with one half)
-            Frag<T> pf[QB];
-#pragma unroll
-            for (int qb = 0; qb < QB; qb++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    pf[qb].v[i] = from_f32<T>(s[2 * c][qb][i]);
-                    pf[qb].v[4 + i] = from_f32<T>(s[2 * c + 1][qb][i]);
-                }
-#pragma unroll
-            for (int d = 0; d < DB; d++) {
-                Frag<T> vf;
-                if constexpr (VT) {
-                    vf = lds_frag8<T>(vt + (d * 16 + fr) * LDV + kc + g * 8);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        vf.v[e] = vt[(kc + 16 * (e >> 2) + 4 * g + (e & 3)) * LDV + d * 16 + fr];
-                }
-#pragma unroll
-                for (int qb = 0; qb < QB; qb++) mma16(o[d][qb], vf, pf[qb]);
             }
         }
         if (tn < ntiles) ATTN_LSTORE(buf ^ 1);
@@ -279,8 +298,23 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
 #undef ATTN_GLOAD
 #undef ATTN_LSTORE
 
-    // The second half's (m, l, O) into the first's, through the K tiles (every wavefront is past
-    // the last tile's barrier).
+    // The second half's (m, l, O) into the first's.
+    auto& o = oh[0];
+    auto& l_run = lh[0];
+    auto merge = [&](int qb, float m1, float l1, auto&& o1) {
+        const float m0 = mh[0][qb], mt = fmaxf(m0, m1), mu = mt == -INFINITY ? 0.f : mt;
+        const float c0 = fast_exp2(m0 - mu), c1 = fast_exp2(m1 - mu);
+#pragma unroll
+        for (int d = 0; d < DB; d++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[d][qb][i] = fmaf(o[d][qb][i], c0, o1(d, i) * c1);
+        l_run[qb] = fmaf(l_run[qb], c0, l1 * c1);
+    };
+    if constexpr (HPW == 2) {
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++) merge(qb, mh[1][qb], lh[1][qb], [&](int d, int i) { return oh[1][d][qb][i]; });
+    }
+    // Through the K tiles (every wavefront is past the last tile's barrier).
     if constexpr (KVS == 2) {
         static_assert(sizeof(Ks) >= sizeof(float) * 4 * 64 * (4 * DB + 2), "merge buffer");
         float* comb = reinterpret_cast<float*>(&Ks[0][0]) + (size_t)wave * 64 * (4 * DB + 2) + lane;
@@ -292,20 +326,12 @@ __global__ __launch_bounds__(256 * kKeyHalves<T>) void attn_kernel(AttnArgs<T> a
                 for (int d = 0; d < DB; d++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) comb[(4 * d + i) * 64] = o[d][qb][i];
-                comb[4 * DB * 64] = m_run[qb];
+                comb[4 * DB * 64] = mh[0][qb];
                 comb[(4 * DB + 1) * 64] = l_run[qb];
             }
             __syncthreads();
-            if (!half) {
-                const float m1 = comb[4 * DB * 64], l1 = comb[(4 * DB + 1) * 64];
-                const float mt = fmaxf(m_run[qb], m1), mu = mt == -INFINITY ? 0.f : mt;
-                const float c0 = fast_exp2(m_run[qb] - mu), c1 = fast_exp2(m1 - mu);
-#pragma unroll
-                for (int d = 0; d < DB; d++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[d][qb][i] = o[d][qb][i] * c0 + comb[(4 * d + i) * 64] * c1;
-                l_run[qb] = l_run[qb] * c0 + l1 * c1;
-            }
+            if (!half)
+                merge(qb, comb[4 * DB * 64], comb[(4 * DB + 1) * 64], [&](int d, int i) { return comb[(4 * d + i) * 64]; });
         }
         if (half) return;
     }
@@ -342,9 +368,9 @@ int launch_q(const AttnArgs<T>& a, int qb, hipStream_t st) {
     int wq = 16 * qb;
     dim3 grid((a.Sq + 4 * wq - 1) / (4 * wq), a.H, a.B);
     if (qb == 1)
-        attn_kernel<T, DH, 1, VT><<<grid, 256 * kKeyHalves<T>, 0, st>>>(a);
+        attn_kernel<T, DH, 1, VT><<<grid, 256 * kKeyWaves<T, DH, 1, VT>, 0, st>>>(a);
     else
-        attn_kernel<T, DH, 2, VT><<<grid, 256 * kKeyHalves<T>, 0, st>>>(a);
+        attn_kernel<T, DH, 2, VT><<<grid, 256 * kKeyWaves<T, DH, 2, VT>, 0, st>>>(a);
     return 0;
 }
 

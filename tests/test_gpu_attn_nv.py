@@ -89,6 +89,28 @@ def test_operands_at_any_element_alignment(dtype, Sq, Skv, Dh):
         assert np.array_equal(g, got[0])
 
 
+@pytest.mark.parametrize("Dh", [64, 128])
+@pytest.mark.parametrize("Skv", [31, 70, 150])
+def test_f32_rows_do_not_depend_on_the_launch_size(Dh, Skv):
+    # Few heads take one query block per wavefront and two wavefronts per tile; many take two query
+    # blocks, and with 64 dims both key halves in one wavefront: the same arithmetic, so the same bits.
+    Sq, many = 130, 300
+    rng = np.random.default_rng(Skv)
+    q, k, v = (torch.from_numpy(rng.standard_normal((1, 1, n, Dh)).astype(np.float32)).to("cuda")
+               for n in (Sq, Skv, Skv))
+    m = torch.ones((1, Skv), device="cuda")
+    m[0, 5:9] = 0
+    got = []
+    for H in (1, many):
+        qq, kk, vv = (a.expand(1, H, -1, -1).contiguous() for a in (q, k, v))
+        out = torch.full((1, H, Sq, Dh), 7.0, dtype=torch.float32, device="cuda")
+        ops.sdpa(L.DTYPE_F32, qq.data_ptr(), kk.data_ptr(), vv.data_ptr(), m.data_ptr(), 1, H, Sq, Skv, Dh, Dh ** -0.5,
+                 out.data_ptr())
+        torch.cuda.synchronize()
+        got.append(out.cpu().numpy()[0])
+    assert np.isfinite(got[0]).all() and np.array_equal(got[1], np.repeat(got[0], many, 0))
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
 @pytest.mark.parametrize("Dh", [64, 128])
 def test_scores_of_minus_infinity(oracle64, dtype, Dh):

@@ -1480,7 +1480,10 @@ void launch_tile_rows(const void* src, int N, int row_bytes, void* dst, hipStrea
 //     W1|W3 launches of more 128x128 tiles than the chip holds at once (512) take 192x128: the same two
 //     workgroups per CU, 1.25x the flops per LDS byte (1500 x 5632 x 1024 28.9 -> 24.2 us; 8 steps
 //     of two chains of 1500 rows 14.6 -> 14.8 ms, 2100 rows 19.6 -> 18.9, 6000 rows 52.8 -> 51.3;
-//     with fewer tiles it loses: 1000 rows 10.1 -> 11.3).
+//     with fewer tiles it loses: 1000 rows 10.1 -> 11.3).  In f32 the MFMAs bound both tiles, and a
+//     launch takes its rounds of 512 workgroups times the tile's size: 192x128 only where that is less (MLP
+//     operator of the same width, 128x128 against 192x128: 1500 rows 289 and 277 us, but 2304 rows 420 and 464, 2800 rows
+//     423 and 536, 4500 rows 694 and 724, 6000 rows 831 and 812).
 //   * The D-wide residual projections: 64x64 in four stages, 32x64 while that still leaves most
 //     CUs one workgroup at most (8 steps at 128 frames 7.79 -> 7.44, 384 frames 8.14 -> 7.80, 512 frames 8.29 ->
 //     8.55), 128x128 in two stages for batches that give two workgroups per CU; in between, where
@@ -1507,8 +1510,11 @@ template <typename T, bool F8>
 static int launch_swiglu(const GemmArgs<T>& a, hipStream_t st) {
     if (tile_count(a.M, a.N, 64, 64) <= 256) return launch_cfg<T, 64, 64, 2, 1, 4, EPI_SWIGLU, F8>(a, st);
     if (tile_count(a.M, a.N, 128, 64) <= 352) return launch_cfg<T, 128, 64, 4, 1, 3, EPI_SWIGLU, F8>(a, st);
-    if constexpr (!F8)
-        if (tile_count(a.M, a.N, 128, 128) > 512) return launch_cfg<T, 192, 128, 2, 2, 2, EPI_SWIGLU>(a, st);
+    if constexpr (!F8) {
+        const long t128 = tile_count(a.M, a.N, 128, 128), t192 = tile_count(a.M, a.N, 192, 128);
+        const bool taller = sizeof(T) == 2 ? t128 > 512 : 3 * ((t192 + 511) / 512) < 2 * ((t128 + 511) / 512);
+        if (taller) return launch_cfg<T, 192, 128, 2, 2, 2, EPI_SWIGLU>(a, st);
+    }
     return launch_cfg<T, 128, 128, 2, 2, 2, EPI_SWIGLU, F8>(a, st);
 }
 // The residual projections (N = the model width): the smallest tile that needs no second round.

@@ -457,13 +457,15 @@ int irodori_op_sdpa(int dtype, const void* q, const void* k, const void* v, cons
                     float* out, void* stream);
 /* No counterpart in the reference: irodori_op_sdpa for callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops that forbid hipMalloc).  Same
- * arguments, kernels and results.  With a 16-bit dtype, head_dim 64 and seq_kv <= 16384 it
- * takes operands of at most IRODORI_SDPA_SCRATCH_BYTES (Q + V^T with its keys rounded up to 64,
- * in the operand dtype, + one key bit each, every part rounded up to 256 bytes; else
- * IRODORI_ERR_SHAPE), `stream` must belong to the current device (else
- * IRODORI_ERR_INVALID_ARG), and the first call on a device, which loads the kernel, must not be
- * made under graph capture (IRODORI_ERR_INVALID_ARG): capturing callers make one call outside
- * the capture first; later calls may be captured and replayed. */
+ * arguments, kernels and results; neither entry point allocates.  With a 16-bit dtype, head_dim
+ * 64 and seq_kv <= 16384 this one takes operands of at most IRODORI_SDPA_SCRATCH_BYTES (Q + V^T
+ * with its keys rounded up to 64, in the operand dtype, + one key bit each, every part rounded
+ * up to 256 bytes; else IRODORI_ERR_SHAPE: a limit of the contract, no buffer of that size
+ * exists), `stream` must belong to the current device (else IRODORI_ERR_INVALID_ARG), and the
+ * first such call on a device, which loads the code of the kernel's 16-bit variants and sets
+ * their LDS limits, must not be made under graph capture (IRODORI_ERR_INVALID_ARG): capturing
+ * callers make one call outside the capture first; later calls may be captured and replayed.
+ * Other shapes and dtypes may be captured from the first call on. */
 #define IRODORI_SDPA_SCRATCH_BYTES (16u << 20)
 int irodori_op_sdpa_noalloc(int dtype, const void* q, const void* k, const void* v, const float* mask,
                             int batch, int heads, int seq_q, int seq_kv, int head_dim, float scale,

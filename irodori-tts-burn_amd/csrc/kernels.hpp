@@ -410,5 +410,7 @@ int launch_attention32(const AttnArgs<bf16>& a, hipStream_t st);
 // out_mode 0 or 1 (kernels_attn_nv.hip).
 template <typename T, int DH>
 int launch_attention_nv(const AttnArgs<T>& a, hipStream_t st);
+// Sets the LDS limits of all its variants on the current device, as each variant's first launch does.
+hipError_t prepare_attention_nv();
 
 }  // namespace irodori

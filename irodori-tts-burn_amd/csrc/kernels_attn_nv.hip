@@ -420,15 +420,29 @@ __global__ __launch_bounds__(64 * QB * KVS) __attribute__((amdgpu_waves_per_eu(1
     }
 }
 
+template <int DH, int KVS>
+constexpr int kLds = 4 * KVS * KT * DH * 2;
+template <typename T, int DH, int QB, int KVS, bool UNAL>
+hipError_t set_limit() {
+    static LdsLimit lim;
+    return set_lds_limit_once(lim, (const void*)attn_nv_kernel<T, DH, QB, KVS, UNAL>, kLds<DH, KVS>);
+}
 template <typename T, int DH, int QB, int KVS, bool UNAL = false>
 int launch_cfg(const AttnArgs<T>& a, hipStream_t st) {
-    constexpr int lds = 4 * KVS * KT * DH * 2;
-    static LdsLimit lim;
-    if (set_lds_limit_once(lim, (const void*)attn_nv_kernel<T, DH, QB, KVS, UNAL>, lds) != hipSuccess) return -2;
+    if (set_limit<T, DH, QB, KVS, UNAL>() != hipSuccess) return -2;
     const long wgs = (long)((a.Sq + 32 * QB - 1) / (32 * QB)) * a.H * a.B;
     if (wgs > 0x7fffffffL) return -1;
-    attn_nv_kernel<T, DH, QB, KVS, UNAL><<<(unsigned)wgs, 64 * QB * KVS, lds, st>>>(a, (a.Sq + 32 * QB - 1) / (32 * QB));
+    attn_nv_kernel<T, DH, QB, KVS, UNAL>
+        <<<(unsigned)wgs, 64 * QB * KVS, kLds<DH, KVS>, st>>>(a, (a.Sq + 32 * QB - 1) / (32 * QB));
     return 0;
+}
+// Every variant that launch_attention_nv<T, DH> chooses from.
+template <typename T, int DH>
+hipError_t set_limits() {
+    hipError_t e = set_limit<T, DH, 2, 2, false>();
+    if (e == hipSuccess) e = set_limit<T, DH, 2, 2, true>();
+    if (DH == 128 && e == hipSuccess) e = set_limit<T, DH, 4, 2, false>();
+    return e;
 }
 
 }  // namespace
@@ -455,5 +469,13 @@ template int launch_attention_nv<bf16, 64>(const AttnArgs<bf16>&, hipStream_t);
 template int launch_attention_nv<bf16, 128>(const AttnArgs<bf16>&, hipStream_t);
 template int launch_attention_nv<f16, 64>(const AttnArgs<f16>&, hipStream_t);
 template int launch_attention_nv<f16, 128>(const AttnArgs<f16>&, hipStream_t);
+
+hipError_t prepare_attention_nv() {
+    hipError_t e = set_limits<bf16, 64>();
+    if (e == hipSuccess) e = set_limits<bf16, 128>();
+    if (e == hipSuccess) e = set_limits<f16, 64>();
+    if (e == hipSuccess) e = set_limits<f16, 128>();
+    return e;
+}
 
 }  // namespace irodori

@@ -50,7 +50,8 @@ int sdpa_run(int dtype, const void* q, const void* k, const void* v, const float
 }
 
 // irodori_op_sdpa_noalloc's contract: 16-bit operands with Dh = 64 and at most 16384 keys are
-// held to IRODORI_SDPA_SCRATCH_BYTES of Q, V^T and key bits.
+// held to IRODORI_SDPA_SCRATCH_BYTES of Q, V^T and key bits.  (The kernels need no such buffer; callers
+// may rely on the refusal.)
 bool noalloc_bounded(int dtype, int Dh, int Skv) { return dtype != IRODORI_DTYPE_F32 && Dh == 64 && Skv <= 16384; }
 size_t noalloc_bytes(int B, int H, int Sq, int Skv) {
     const size_t vs = (size_t)(Skv + 63) / 64 * 64;
@@ -59,10 +60,10 @@ size_t noalloc_bytes(int B, int H, int Sq, int Skv) {
 }
 
 constexpr int kMaxDevices = 64;
-std::atomic<bool> g_called[kMaxDevices] = {};
+std::atomic<bool> g_prepared[kMaxDevices] = {};
 
-// The stream must be the current device's, and a device's first call (which loads the kernel's
-// code and sets its LDS limit) must not be captured: capturing callers make one eager call first.
+// The stream must be the current device's, and a device's first call must not be captured: it loads
+// the code of the row-major kernel's variants and sets their LDS limits, so that no later call, captured or not, does.
 int check_noalloc_stream(hipStream_t st) {
     int dev = -1;
     IRO_HIP_CHECK(hipGetDevice(&dev));
@@ -74,13 +75,14 @@ int check_noalloc_stream(hipStream_t st) {
                         " but device " + std::to_string(dev) + " is current; make the stream's device current");
     }
     IRO_REQUIRE(dev >= 0 && dev < kMaxDevices, IRODORI_ERR_INVALID_ARG, "device index beyond the device table");
-    if (!g_called[dev].load()) {
+    if (!g_prepared[dev].load()) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         IRO_HIP_CHECK(hipStreamIsCapturing(st, &cs));
         IRO_REQUIRE(cs == hipStreamCaptureStatusNone, IRODORI_ERR_INVALID_ARG,
                     "irodori_op_sdpa_noalloc: the first call on a device must not be under graph capture; make "
                     "one call outside the capture first");
-        g_called[dev].store(true);
+        IRO_HIP_CHECK(prepare_attention_nv());
+        g_prepared[dev].store(true);
     }
     return IRODORI_OK;
 }

@@ -1,8 +1,11 @@
 """irodori_op_sdpa_noalloc (no counterpart in the reference; for callers that cannot
-allocate): the same kernels as irodori_op_sdpa, the staging in the library's fixed per-GPU
-buffer.  Checked against irodori_op_sdpa through the C ABI on two calls in a row (the
-second smaller, so the first call's staging is still in the buffer), bit for bit (same
-kernels, same inputs), and against the oracle; shapes beyond the buffer are refused."""
+allocate): the same kernels as irodori_op_sdpa, without device memory of their own.  Checked
+against irodori_op_sdpa through the C ABI, bit for bit (same kernels, same inputs), and
+against the oracle; shapes beyond the contract's size limit and a captured first call are refused."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -50,9 +53,9 @@ def test_noalloc_matches_allocating_entry_point(oracle64, dtype, tdt):
 
 
 def _boundary_shape(sq):
-    # One head of 64 keys: the staging is Q (sq x 128 bytes, rounded up to 256) + V^T
-    # (8192 bytes) + the key bits (one word, rounded up to 256).  sq = 131006 fills the
-    # 16 MiB buffer exactly; 131007 is one 256-byte step past it.
+    # One head of 64 keys: the contract counts Q (sq x 128 bytes, rounded up to 256) + V^T
+    # (8192 bytes) + the key bits (one word, rounded up to 256).  sq = 131006 is
+    # 16 MiB exactly; 131007 is one 256-byte step past it.
     return 1, 1, sq, 64
 
 
@@ -77,7 +80,7 @@ def test_noalloc_refuses_shapes_beyond_its_buffer():
 
 
 def test_noalloc_under_graph_capture_replays_the_eager_result():
-    # One eager call (it resolves the buffer's address), then the same call captured in a
+    # One eager call (it loads the kernels), then the same call captured in a
     # graph on torch's capture stream and replayed several times, with eager work on the
     # same buffers between the replays; every replay rewrites the output bit for bit.
     B, H, Sq, Skv = 2, 4, 200, 300
@@ -100,9 +103,57 @@ def test_noalloc_under_graph_capture_replays_the_eager_result():
     other_q, other_k, other_v, other_m = _inputs(1, 2, 50, 70, 6)
     for rep in range(4):
         out.fill_(7.0)
-        # An eager call of another shape in between leaves other contents in the buffer.
+        # An eager call of another shape in between.
         _run(ops.sdpa_noalloc, L.DTYPE_BF16, torch.bfloat16, other_q, other_k, other_v, other_m)
         g.replay()
         torch.cuda.synchronize()
         assert np.array_equal(out.cpu().numpy(), eager), rep
 
+
+CHILD = """
+import torch
+from irodori_hip import _lib as L, ops
+from irodori_hip.config import IrodoriError
+
+def captured(code, dtype, dh, off):
+    q = torch.randn(2 * 40 * dh + off, device="cuda").to(dtype)[off:]
+    out = torch.zeros(2 * 40 * dh, device="cuda")
+    call = lambda: ops.sdpa_noalloc(code, q.data_ptr(), q.data_ptr(), q.data_ptr(), 0, 1, 2, 40, 40, dh, 0.125,
+                                    out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call()
+    got = []
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        got.append(out.clone())
+    call()
+    torch.cuda.synchronize()
+    assert out.abs().sum() > 0 and all(torch.equal(a, out) for a in got)
+    return call
+
+captured(L.DTYPE_BF16, torch.bfloat16, 128, 0)  # outside the contract's first-call rule
+try:
+    captured(L.DTYPE_BF16, torch.bfloat16, 64, 0)
+    raise SystemExit("a captured first call was accepted")
+except IrodoriError as e:
+    assert e.kind == "InvalidArg", e.kind
+x = torch.randn(4 * 64, device="cuda").to(torch.bfloat16)
+o = torch.empty(4 * 64, device="cuda")
+ops.sdpa_noalloc(L.DTYPE_BF16, x.data_ptr(), x.data_ptr(), x.data_ptr(), 0, 1, 1, 4, 4, 64, 0.125, o.data_ptr(), 0)
+torch.cuda.synchronize()
+for code, dtype in ((L.DTYPE_F16, torch.float16), (L.DTYPE_BF16, torch.bfloat16)):
+    for off in (0, 1):
+        captured(code, dtype, 64, off)
+print("captures ok")
+"""
+
+
+def test_first_call_rule_in_a_fresh_process():
+    # The first call's state is the process's, so the rule needs a process of its own: a captured first
+    # call is refused, and one eager call of any 64-dim 16-bit shape prepares every variant for capture.
+    env = dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(L.__file__)))
+    r = subprocess.run([sys.executable, "-W", "ignore", "-c", CHILD], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "captures ok" in r.stdout, r.stdout + r.stderr

@@ -27,7 +27,6 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(bf16 v) { return static_cast<float>(v); }
-__device__ __forceinline__ float to_f32(f16 v) { return static_cast<float>(v); }
 
 template <typename T>
 __device__ __forceinline__ T from_f32(float v);
@@ -35,8 +34,6 @@ template <>
 __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <>
 __device__ __forceinline__ bf16 from_f32<bf16>(float v) { return static_cast<bf16>(v); }
-template <>
-__device__ __forceinline__ f16 from_f32<f16>(float v) { return static_cast<f16>(v); }
 
 // Snake1d (codec/layers.rs:24-31): v + sin(a v)^2 / (a + 1e-9), from the channel's
 // constants (a, ar = a / pi, hc = 0.5 / (a + 1e-9)).  For bf16 results (rounded to 8 bits)
@@ -106,30 +103,13 @@ template <>
 struct Frag<float> {
     f32x8 v;
 };
-template <>
-struct Frag<f16> {
-    f16x8 v;
-};
 
 __device__ __forceinline__ void mma16(f32x4& acc, const Frag<bf16>& a, const Frag<bf16>& b) {
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc, 0, 0, 0);
 }
-__device__ __forceinline__ void mma16(f32x4& acc, const Frag<f16>& a, const Frag<f16>& b) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v, b.v, acc, 0, 0, 0);
-}
 __device__ __forceinline__ void mma16(f32x4& acc, const Frag<float>& a, const Frag<float>& b) {
 #pragma unroll
     for (int j = 0; j < 8; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.v[j], b.v[j], acc, 0, 0, 0);
-}
-
-// 16-byte vector loads/stores.
-template <typename V>
-__device__ __forceinline__ V ld_vec(const void* p) {
-    return *reinterpret_cast<const V*>(p);
-}
-template <typename V>
-__device__ __forceinline__ void st_vec(void* p, const V& v) {
-    *reinterpret_cast<V*>(p) = v;
 }
 
 // Load a k32 fragment (8 contiguous elements) from LDS or global memory.
@@ -145,12 +125,6 @@ template <>
 __device__ __forceinline__ Frag<float> load_frag<float>(const float* p) {
     Frag<float> f;
     f.v = *reinterpret_cast<const f32x8*>(p);
-    return f;
-}
-template <>
-__device__ __forceinline__ Frag<f16> load_frag<f16>(const f16* p) {
-    Frag<f16> f;
-    f.v = *reinterpret_cast<const f16x8*>(p);
     return f;
 }
 

@@ -448,8 +448,7 @@ struct PartOpts {
 
 // One kernel of a DiT block over batch rows [r0, r0 + B) of the context's buffers, on
 // stream st.  Every row-indexed buffer is offset to row r0; mt must map the slice's local
-// row b to the vector of global row r0 + b (rows_per_vec == 1 with the table offset, or
-// all rows sharing one vector).
+// row b to the vector of global row r0 + b (r0 == 0, or all rows sharing one vector).
 template <typename T>
 int enqueue_part(irodori_ctx* c, int l, int B, int S, const ModTable& mt, int part, int r0,
                  hipStream_t st, const PartOpts& opt = PartOpts()) {

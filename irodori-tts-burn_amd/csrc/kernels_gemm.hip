@@ -10,7 +10,7 @@
 //     256-byte bank line, so rows 2p and 2p+1 use the same xor key).
 //   * v_mfma_f32_32x32x16_bf16 (the full-rate bf16 shape on gfx950; 16x16x32 issues at
 //     half rate) on 32x32 blocks; the f32 path uses v_mfma_f32_32x32x2_f32 on the same
-//     fragments.  4 wavefronts per workgroup in a 2x2 grid.
+//     fragments.  Two, four or eight wavefronts per workgroup in a grid (WAVES_M x WAVES_N).
 //   * Workgroup barriers are raw s_barrier after an explicit vmcnt wait for the slice
 //     being consumed, so later slices stay in flight across the barrier.
 //
@@ -267,13 +267,9 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
     const __amdgpu_buffer_rsrc_t rA = make_rsrc(Ab + (size_t)m0 * lda * ES, (unsigned)((size_t)arows * lda * ES));
     // W row rr of the tile: group rr / 64 at 64 K ES bytes in either layout; within the
     // group rows are K ES bytes apart (row-major) or 128 (tile-major, where consecutive
-    // slices are 8 KB apart instead of 128 bytes).  A 32-wide tile is one half of a group.
+    // slices are 8 KB apart instead of 128 bytes).
     const bool wt = !CONV && a.w_tiled;
-    constexpr int BN64 = BN < 64 ? 64 : BN;
-    const int ng = n0 / BN64 * BN64;
-    const size_t w_bytes = (size_t)BN64 * K * ES;
-    const size_t w_skip = (size_t)(n0 - ng) * (wt ? 128 : (size_t)K * ES);
-    const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wb + (size_t)ng * K * ES + w_skip, (unsigned)(w_bytes - w_skip));
+    const __amdgpu_buffer_rsrc_t rW = make_rsrc(Wb + (size_t)n0 * K * ES, (unsigned)((size_t)BN * K * ES));
     const unsigned w_row = wt ? 128u : (unsigned)(K * ES), w_slice = wt ? 8192u : 128u;
     unsigned voff[LPW];
 #pragma unroll
@@ -394,8 +390,8 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
 
     // Fused adaLN consumer: lane l of a wave loads the K/32 partial sums of rows m0 + wm0 + l
     // (+ 64) and this wave's shift-bias columns before the operand stream starts, so their
-    // latency hides behind it; iteration 0 of the main loop turns the sums into r = rsqrt(mean
-    // x^2 + eps), kept in registers until the stage buffers are free after the main loop.
+    // latency hides behind it; while the first slices are in flight the sums become r =
+    // rsqrt(mean x^2 + eps), kept in registers until the stage buffers are free after the main loop.
     constexpr bool FUSE_IN = !F8 && (EPI == EPI_QKVG || EPI == EPI_SWIGLU);
     constexpr int RPL = (WM + 63) / 64;  // rows of the wave per lane
     [[maybe_unused]] float4 rsv[RPL][16];
@@ -533,7 +529,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
     constexpr int RD = (F8 ? 2 : 1) * (FM + FN);  // LDS reads of a step
     // MORE: slice kt + STAGES - 1 is loaded during this one; LAST: the last slice.  During the
     // last slice the tile's RoPE rows (QKVG) stream into the stage after it, which was last read
-    // in slice nk - 2: every wave is past that.
+    // in slice nk - STAGES: every wave is past that.
     auto slice = [&](auto more_c, auto last_c, int kt) {
         constexpr bool MORE = decltype(more_c)::value, LAST = decltype(last_c)::value;
         const int stn = st + 1 == STAGES ? 0 : st + 1, stl = st == 0 ? STAGES - 1 : st - 1;
@@ -1419,8 +1415,7 @@ int launch_cfg(const GemmArgs<T>& a, hipStream_t st) {
                  a.next_layer >= a.mt.layers || a.next_kind < 0 || a.next_kind > 1))
         return -1;
     if ((size_t)BN * a.K * ES > 0xffffffffull || (size_t)BM * a.K * ES > 0xffffffffull) return -1;
-    if (a.w_tiled && (CONV || (BN % 64 != 0 && BN != 32) || a.N % 64 != 0)) return -1;
-    if (BN < 64 && a.N % 64 != 0) return -1;  // the weight resource spans whole 64-row groups
+    if (a.w_tiled && (CONV || BN % 64 != 0)) return -1;
     if (CONV) {
         // conv_cp a multiple of half a slice (a slice straddles at most two taps, at its
         // middle); K = the taps' span rounded up to whole slices.
@@ -1471,12 +1466,16 @@ void launch_tile_rows(const void* src, int N, int row_bytes, void* dst, hipStrea
 // has for the 256 CUs and how much of its time is the chain of slices in each:
 //   * Large launches: 128x128 tiles in two stages, two workgroups per CU; with 2x2 wavefronts
 //     of 32x32 blocks the LDS traffic is 1.5x the MFMA time (3x for 64x64).
-//   * Launches that leave CUs idle at that size (one utterance's rows at N = 4 D or 2 F) take
-//     smaller tiles in three or four stages with the pipelined loop, more workgroups and
+//   * Launches of few such tiles (one utterance's rows at N = 4 D or 2 F) take smaller tiles in three or four stages with the pipelined loop, more workgroups and
 //     shorter slices.  8 steps of the d1024 sampler, ms, with QKV+gate tiles / W1|W3 tiles of
 //     128x128 -> the choice below: 24 frames 8.30 -> 7.08, 128 frames 8.14 -> 6.01, 256 frames 7.92 ->
 //     6.49, 384 frames 8.14 -> 7.06, 512 frames 8.29 -> 7.90, 640 frames 8.89 -> 8.60; at 750 and beyond
-//     128x128 is the better one (40 steps 45.5 against 45.8 and 47.0 ms).
+//     128x128 is the better one (40 steps 45.5 against 45.8 and 47.0 ms).  The lines (64x64 up to
+//     256 tiles, 64x128 up to 320 and 128x64 up to 352, which are 128x128 launches of up to 160 and
+//     176) come from these bf16 runs, whose chains share the CUs.  Alone on the chip at 512 rows, chosen tile
+//     against 128x128: bf16 QKV+gate 10.8 and 15.5 us, W1|W3 11.8 and 13.2; fp8 8.6 and 12.1, 8.7 and
+//     10.2; an f32 forward of four layers 1133 and 1326 us, 1222; no type loses at 64 to 1024 rows (there the
+//     small tiles would win up to 1024 rows in f32, and QKV+gate in fp8).
 //     W1|W3 launches of more 128x128 tiles than the chip holds at once (512) take 192x128: the same two
 //     workgroups per CU, 1.25x the flops per LDS byte (1500 x 5632 x 1024 28.9 -> 24.2 us; 8 steps
 //     of two chains of 1500 rows 14.6 -> 14.8 ms, 2100 rows 19.6 -> 18.9, 6000 rows 52.8 -> 51.3;
@@ -1484,9 +1483,9 @@ void launch_tile_rows(const void* src, int N, int row_bytes, void* dst, hipStrea
 //     launch takes its rounds of 512 workgroups times the tile's size: 192x128 only where that is less (MLP
 //     operator of the same width, 128x128 against 192x128: 1500 rows 289 and 277 us, but 2304 rows 420 and 464, 2800 rows
 //     423 and 536, 4500 rows 694 and 724, 6000 rows 831 and 812).
-//   * The D-wide residual projections: 64x64 in four stages, 32x64 while that still leaves most
-//     CUs one workgroup at most (8 steps at 128 frames 7.79 -> 7.44, 384 frames 8.14 -> 7.80, 512 frames 8.29 ->
-//     8.55), 128x128 in two stages for batches that give two workgroups per CU; in between, where
+//   * The D-wide residual projections: 64x64 in four stages, 32x64 up to 192 tiles (8 steps at 128
+//     frames 7.79 -> 7.44, 384 frames, the line, 8.14 -> 7.80, but 512 frames 8.29 -> 8.55; alone on the chip in bf16 the
+//     same time, W2 in fp8 9.6 -> 10.3 us), 128x128 in two stages for batches that give two workgroups per CU; in between, where
 //     those tiles are at most one per CU and leave under half of them idle, 128x128 over eight wavefronts in four
 //     stages (3000 x 1024 x 2816 29.5 -> 21.7 us; two chains of 2250 rows 21.1 -> 20.2 ms per 8 steps).
 //     The encoder's (one stream) also take 128x64 over eight wavefronts (1024 x 1280 x 3328 26.6 ->

@@ -90,8 +90,8 @@ def test_sdpa_op_bf16(oracle64, B, H, Sq, Skv, Dh, mask):
 
 # The reference's f16-input FA tests (fused_sdpa_native_f16.rs:455-585): shapes, masks and
 # tolerances (1e-3 max abs; 1e-6 for the all-masked case), with the oracle fed the same
-# f16-rounded inputs as the reference's own CPU check (:384-388).  head_dim 128 runs on the
-# generic flash kernel, head_dim 64 on the model's joint attention kernel after staging.
+# f16-rounded inputs as the reference's own CPU check (:384-388), on the row-major flash kernel
+# at both head widths.
 F16_CASES = [
     (1, 2, 4, 6, 128, None, 1e-3),
     (1, 2, 4, 8, 128, [1, 1, 1, 1, 1, 0, 0, 0], 1e-3),
@@ -121,9 +121,9 @@ def test_sdpa_op_f16(oracle64, B, H, Sq, Skv, Dh, mask, tol):
     assert np.abs(out.cpu().numpy() - want).max() < tol
 
 
-def test_sdpa_op_f16_bf16_share_the_joint_kernel(oracle64):
-    # Dh = 64 16-bit operators run the model's joint attention kernel: a context longer than
-    # one key tile per parity and a query count that is not a multiple of the query block.
+def test_sdpa_op_f16_bf16_beyond_one_tile_per_parity(oracle64):
+    # Dh = 64 16-bit operators (the row-major kernel): a context longer than one key tile per
+    # parity and a query count that is not a multiple of the query block.
     B, H, Sq, Skv, Dh = 1, 4, 75, 300, 64
     rng = np.random.default_rng(3)
     q, k, v = (rng.standard_normal((B, H, n, Dh)).astype(np.float32) for n in (Sq, Skv, Skv))
@@ -163,7 +163,7 @@ def test_sdpa_config2_joint_shape(oracle64, dtype):
     # Isolated joint attention: B=2, H=16, Dh=64, 750 queries; keys = 750 latent ++ 256 text ++
     # 375 speaker, text valid length uniform in [32, 256], Q/K/V ~ N(0, 1).  (RoPE is part
     # of the model path and is covered by the model tests.)  The oracle takes the same
-    # rounded operands; the kernel also rounds q * scale * log2(e) and P to the operand type.
+    # rounded operands; the kernel also rounds P to the operand type.
     B, H, Sq, Dh, Tt, Ts = 2, 16, 750, 64, 256, 375
     Skv = Sq + Tt + Ts
     rng = np.random.default_rng(0)
@@ -192,8 +192,8 @@ def test_sdpa_config2_joint_shape(oracle64, dtype):
 
 @pytest.mark.parametrize("Skv", [4097, 4796, 16384])
 def test_sdpa_key_tiles_beyond_one_list_word(oracle64, Skv):
-    # More than 64 key tiles per row: the joint kernel's tile list spans several words per
-    # lane.  Row 0 drops whole tiles from the first word (and, when present, the second)
+    # More than 64 key tiles per row: the row-major kernel takes its tile list in several
+    # words.  Row 0 drops whole tiles from the first word (and, when present, the second)
     # so that the entries of later words shift down; row 1 has a partial mask in every tile.
     B, H, Sq, Dh = 2, 2, 70, 64
     rng = np.random.default_rng(Skv)

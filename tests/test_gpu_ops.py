@@ -169,3 +169,32 @@ def test_swiglu_mlp_op_rows_on_their_own_vectors(oracle64, backend, B, S):
     m = oracle64.swiglu(h, w.blocks[0]["w13"], w.blocks[0]["w2"]).reshape(B, S, D).astype(np.float64)
     ref = x + gate[:, None, :].astype(np.float64) * m
     assert rel_l2(got, ref) < TOL[backend] and rel_l2(got - x, ref - x) < 2 * TOL[backend]
+
+
+@pytest.mark.parametrize("backend", [F32, BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("T", [4097, 4796, 16200])
+def test_joint_attention_op_key_tiles_beyond_one_list_word(oracle64, backend, T):
+    # More than 64 context key tiles: the bf16 kernel's tile list spans several words per lane.  Row 0
+    # drops whole tiles from the first word (and, when present, later ones) so that later entries shift
+    # down; row 1 has a partial mask in every tile.
+    cfg = dataclasses.replace(ih.cfg_tiny(), num_layers=1)
+    w = ih.DitWeights.random(cfg, 7, norm_jitter=0.1)
+    B, S, H, Dh = 2, 70, cfg.num_heads, cfg.head_dim
+    rng = np.random.default_rng(T)
+    ctx = ih.ContextKV(*(rng.standard_normal((1, B, T, H, Dh)).astype(np.float32) for _ in range(2)),
+                       np.ones((B, T), np.uint8))
+    ctx.mask[0, 640:1600] = 0
+    ctx.mask[0, 4160:4300] = 0
+    ctx.mask[0, 9000:9999] = 0
+    ctx.mask[1, ::7] = 0
+    ops = [rng.standard_normal((B, S, H, Dh)).astype(np.float32) for _ in range(3)]
+    ops.append(rng.standard_normal((B, S, H * Dh)).astype(np.float32))
+    bufs = [dev(a) for a in ops]
+    out = torch.full((B, S, H * Dh), 7.0, dtype=torch.float32, device="cuda")
+    with ih.HipInferenceEngine(cfg, backend, max_rows=B, max_seq=S, max_ctx=T) as e:
+        e.load_weights(w)
+        e.set_context_kv(ctx)
+        e.joint_attention(0, B, S, *(b.data_ptr() for b in bufs), out.data_ptr())
+        torch.cuda.synchronize()
+    ref = joint_attention_ref(oracle64, cfg, w.blocks[0], *ops, ctx.k[0], ctx.v[0], ctx.mask)
+    assert rel_l2(out.cpu().numpy(), ref) < TOL[backend]

@@ -1,7 +1,7 @@
-// HBM-bound row kernels: RMSNorm, adaLN modulation, in_proj + modulation, output head.
-// One wavefront per row, 4 rows per
-// 256-thread workgroup; rows are read with 16-byte loads and reduced in registers with
-// cross-lane shuffles (no LDS), so each row is read from HBM exactly once.
+// Row kernels: RMSNorm, adaLN modulation, in_proj + modulation, output head.  One wavefront per
+// row, 4 rows per 256-thread workgroup, reduced with cross-lane shuffles.  The model's kernels read
+// a row once with 16-byte loads and keep it in registers; the two operator entry points'
+// (any D) read it twice, four bytes a lane.
 #include "common.hpp"
 #include "kernels.hpp"
 

@@ -667,16 +667,19 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
     };
     // The f32 residual x of the ADD and RESUNIT epilogues, XB rows a batch: the loads of a batch go
     // out before the stores of the one before it, since a wait for loads also waits for every older
-    // store.
-    constexpr int XB = 8, NXB = FM * 16 / XB;
-    [[maybe_unused]] float xv[WINDOWED ? 2 : 1][WINDOWED ? XB : 1][FN];
+    // store.  Not in the f32 unit: its batches (a sinf per element) stay a loop, in which two alternating
+    // buffers would live in scratch memory (128x192 tiles over 249600 frames 2828 us, 2664 without, and 2697
+    // with the same batches of four before the windows).
+    constexpr bool AHEAD = EPI != EPI_RESUNIT || sizeof(T) == 2;
+    constexpr int XB = AHEAD ? 8 : 4, NXB = FM * 16 / XB;
+    [[maybe_unused]] float xv[WINDOWED && AHEAD ? 2 : 1][WINDOWED ? XB : 1][FN];
     [[maybe_unused]] auto load_x = [&](const __amdgpu_buffer_rsrc_t r, int bt) {
         if constexpr (WINDOWED)
 #pragma unroll
             for (int e = 0; e < XB; e++)
 #pragma unroll
                 for (int j = 0; j < FN; j++)
-                    xv[bt & 1][e][j] = __builtin_bit_cast(
+                    xv[AHEAD ? bt & 1 : 0][e][j] = __builtin_bit_cast(
                         float, __builtin_amdgcn_raw_buffer_load_b32(
                                    r, win_elem(bt * XB / 16, bt * XB % 16 + e, j) * 4u, 0, 0));
     };
@@ -811,7 +814,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
         for (int kt2 = 0; kt2 < NK2; kt2++) {
             wait_vmcnt<0>();
             __syncthreads();  // W2 slice kt2 has landed; the s tile is complete
-            if (kt2 == NK2 - 1) load_x(rx, 0);  // behind the last slice's MFMAs
+            if (AHEAD && kt2 == NK2 - 1) load_x(rx, 0);  // behind the last slice's MFMAs
             const unsigned char* at = tl + kt2 * BM * 128;
 #pragma unroll
             for (int ks = 0; ks < KS; ks++) {
@@ -849,13 +852,13 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N == 4 ? 2 : 1))) void gemm_k
             if constexpr (decltype(next_c)::value) ru = win(a.U, win_elems);
 #pragma unroll
             for (int bt = 0; bt < NXB; bt++) {
-                if (bt + 1 < NXB) load_x(rx, bt + 1);
+                if (!AHEAD || bt + 1 < NXB) load_x(rx, AHEAD ? bt + 1 : bt);
 #pragma unroll
                 for (int e = 0; e < XB; e++)
 #pragma unroll
                     for (int j = 0; j < FN; j++) {
                         const int i = bt * XB / 16, ei = bt * XB % 16 + e;
-                        const float v = xv[bt & 1][e][j] + (acc[i][j][ei] + b2[j]);
+                        const float v = xv[AHEAD ? bt & 1 : 0][e][j] + (acc[i][j][ei] + b2[j]);
                         buf_store(v, rx, win_elem(i, ei, j));
                         if constexpr (decltype(next_c)::value)
                             buf_store(from_f32<T>(snake_eval<T>(v, a2[j], ar2[j], hc2[j])), ru, win_elem(i, ei, j));

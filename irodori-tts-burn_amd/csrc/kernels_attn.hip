@@ -48,14 +48,15 @@ __device__ __forceinline__ Frag<float> lds_frag8<float>(const float* p) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// f32: the two halves of a tile's keys keep their own softmax state (kKeyHalves), merged at the end.
-// They go to separate wavefronts (kKeyWaves), so that every SIMD has a second one to run its MFMAs
-// (32 cycles each) while the first is in its softmax or waits for LDS; with one per SIMD the 41 k
-// MFMA cycles of a 64-query workgroup at 631 keys took 100 k.  Two query blocks of 64 dims on
-// row-major V (launches that fill the chip) leave one wavefront enough to interleave, which then takes both
-// halves, in the same arithmetic and without the merge through LDS: 16 x 16 heads x 750 x 1381 658 -> 602 us, 4 x
-// 32 x 500 x 70 33.2 -> 28.0.  On V^T with its second segment that order is mixed (joint operator, 16 x
-// 512 tokens 268 -> 249 us, but 6 x 700 217 -> 253, 8 x 750 255 -> 286), and for 128 dims it lacks the registers.
+// f32: the two halves of a tile's keys keep their own softmax state (kKeyHalves), merged at the
+// end. They go to separate wavefronts (kKeyWaves), so that every SIMD has a second one to run its
+// MFMAs (32 cycles each) while the first is in its softmax or waits for LDS; with one per SIMD the
+// 41 k MFMA cycles of a 64-query workgroup at 631 keys took 100 k.  Two query blocks of 64 dims on
+// row-major V (launches that fill the chip) leave one wavefront enough to interleave, which then
+// takes both halves, in the same arithmetic and without the merge through LDS: 16 x 16 heads x 750
+// x 1381 658 -> 602 us, 4 x 32 x 500 x 70 33.2 -> 28.0.  On V^T with its second segment that order
+// is mixed (joint operator, 16 x 512 tokens 268 -> 249 us, but 6 x 700 217 -> 253, 8 x 750 255 ->
+// 286), and for 128 dims it lacks the registers.
 template <typename T>
 constexpr int kKeyHalves = sizeof(T) == 4 ? 2 : 1;
 template <typename T, int DH, int QB, bool VT>

@@ -19,7 +19,7 @@
 //
 // What bounds it: with about one wavefront per SIMD, a tile step's chain of barrier, LDS reads,
 // 32 quarter-rate exponentials and ~90 other VALU operations, and the P V MFMAs.  At the
-// published model's call (1 x 20 heads, 750 queries, 950 keys of which 80 % valid, 64-dim): 13.2
+// published model's call (1 x 20 heads, 750 queries, 950 keys of which 80 % valid, 64-dim): 12.1
 // us back to back, where staging Q, V^T and the key bits in a buffer allocated per call took 8.0
 // us before a 9.9 us attention (30 us a call with the allocation and the gap); 1 x 10 x 256 x 256
 // at 128-dim 9.5 against 21.8 us on 16x16 tiles with one 16-query block per wavefront.

@@ -1469,30 +1469,33 @@ void launch_tile_rows(const void* src, int N, int row_bytes, void* dst, hipStrea
 // has for the 256 CUs and how much of its time is the chain of slices in each:
 //   * Large launches: 128x128 tiles in two stages, two workgroups per CU; with 2x2 wavefronts
 //     of 32x32 blocks the LDS traffic is 1.5x the MFMA time (3x for 64x64).
-//   * Launches of few such tiles (one utterance's rows at N = 4 D or 2 F) take smaller tiles in three or four stages with the pipelined loop, more workgroups and
-//     shorter slices.  8 steps of the d1024 sampler, ms, with QKV+gate tiles / W1|W3 tiles of
-//     128x128 -> the choice below: 24 frames 8.30 -> 7.08, 128 frames 8.14 -> 6.01, 256 frames 7.92 ->
-//     6.49, 384 frames 8.14 -> 7.06, 512 frames 8.29 -> 7.90, 640 frames 8.89 -> 8.60; at 750 and beyond
-//     128x128 is the better one (40 steps 45.5 against 45.8 and 47.0 ms).  The lines (64x64 up to
-//     256 tiles, 64x128 up to 320 and 128x64 up to 352, which are 128x128 launches of up to 160 and
-//     176) come from these bf16 runs, whose chains share the CUs.  Alone on the chip at 512 rows, chosen tile
-//     against 128x128: bf16 QKV+gate 10.8 and 15.5 us, W1|W3 11.8 and 13.2; fp8 8.6 and 12.1, 8.7 and
-//     10.2; an f32 forward of four layers 1133 and 1326 us, 1222; no type loses at 64 to 1024 rows (there the
-//     small tiles would win up to 1024 rows in f32, and QKV+gate in fp8).
-//     W1|W3 launches of more 128x128 tiles than the chip holds at once (512) take 192x128: the same two
-//     workgroups per CU, 1.25x the flops per LDS byte (1500 x 5632 x 1024 28.9 -> 24.2 us; 8 steps
-//     of two chains of 1500 rows 14.6 -> 14.8 ms, 2100 rows 19.6 -> 18.9, 6000 rows 52.8 -> 51.3;
-//     with fewer tiles it loses: 1000 rows 10.1 -> 11.3).  In f32 the MFMAs bound both tiles, and a
-//     launch takes its rounds of 512 workgroups times the tile's size: 192x128 only where that is less (MLP
-//     operator of the same width, 128x128 against 192x128: 1500 rows 289 and 277 us, but 2304 rows 420 and 464, 2800 rows
-//     423 and 536, 4500 rows 694 and 724, 6000 rows 831 and 812).
+//   * Launches of few such tiles (one utterance's rows at N = 4 D or 2 F) take smaller tiles in
+//     three or four stages with the pipelined loop, more workgroups and shorter slices.  8 steps of
+//     the d1024 sampler, ms, with QKV+gate tiles / W1|W3 tiles of 128x128 -> the choice below: 24
+//     frames 8.30 -> 7.08, 128 frames 8.14 -> 6.01, 256 frames 7.92 -> 6.49, 384 frames 8.14 ->
+//     7.06, 512 frames 8.29 -> 7.90, 640 frames 8.89 -> 8.60; at 750 and beyond 128x128 is the
+//     better one (40 steps 45.5 against 45.8 and 47.0 ms).  The lines (64x64 up to 256 tiles,
+//     64x128 up to 320 and 128x64 up to 352, which are 128x128 launches of up to 160 and 176) come
+//     from these bf16 runs, whose chains share the CUs.  Alone on the chip at 512 rows, chosen tile
+//     against 128x128: bf16 QKV+gate 10.8 and 15.5 us, W1|W3 11.8 and 13.2; fp8 8.6 and 12.1, 8.7
+//     and 10.2; an f32 forward of four layers 1133 and 1326 us, 1222; no type loses at 64 to 1024
+//     rows (there the small tiles would win up to 1024 rows in f32, and QKV+gate in fp8).
+//     W1|W3 launches of more 128x128 tiles than the chip holds at once (512) take 192x128: the same
+//     two workgroups per CU, 1.25x the flops per LDS byte (1500 x 5632 x 1024 28.9 -> 24.2 us; 8
+//     steps of two chains of 1500 rows 14.6 -> 14.8 ms, 2100 rows 19.6 -> 18.9, 6000 rows 52.8 ->
+//     51.3; with fewer tiles it loses: 1000 rows 10.1 -> 11.3).  In f32 the MFMAs bound both tiles,
+//     and a launch takes its rounds of 512 workgroups times the tile's size: 192x128 only where
+//     that is less (MLP operator of the same width, 128x128 against 192x128: 1500 rows 289 and 277
+//     us, but 2304 rows 420 and 464, 2800 rows 423 and 536, 4500 rows 694 and 724, 6000 rows 831
+//     and 812).
 //   * The D-wide residual projections: 64x64 in four stages, 32x64 up to 192 tiles (8 steps at 128
-//     frames 7.79 -> 7.44, 384 frames, the line, 8.14 -> 7.80, but 512 frames 8.29 -> 8.55; alone on the chip in bf16 the
-//     same time, W2 in fp8 9.6 -> 10.3 us), 128x128 in two stages for batches that give two workgroups per CU; in between, where
-//     those tiles are at most one per CU and leave under half of them idle, 128x128 over eight wavefronts in four
-//     stages (3000 x 1024 x 2816 29.5 -> 21.7 us; two chains of 2250 rows 21.1 -> 20.2 ms per 8 steps).
-//     The encoder's (one stream) also take 128x64 over eight wavefronts (1024 x 1280 x 3328 26.6 ->
-//     21.9 us; in two chains of 1500 rows, which share the CUs, that tile costs 4 %).
+//     frames 7.79 -> 7.44, 384 frames, the line, 8.14 -> 7.80, but 512 frames 8.29 -> 8.55; alone
+//     on the chip in bf16 the same time, W2 in fp8 9.6 -> 10.3 us), 128x128 in two stages for
+//     batches that give two workgroups per CU; in between, where those tiles are at most one per CU
+//     and leave under half of them idle, 128x128 over eight wavefronts in four stages (3000 x 1024
+//     x 2816 29.5 -> 21.7 us; two chains of 2250 rows 21.1 -> 20.2 ms per 8 steps). The encoder's
+//     (one stream) also take 128x64 over eight wavefronts (1024 x 1280 x 3328 26.6 -> 21.9 us; in
+//     two chains of 1500 rows, which share the CUs, that tile costs 4 %).
 //   * f32 stores (the encoder's QKV+gate, the shift biases): 64x128 over eight wavefronts where
 //     64x64 needs a second round and it does not (256 x 5120 x 1280 13.2 -> 11.2 us).
 template <typename T>
